@@ -2,8 +2,6 @@
 // the Q parity entry: tile geometry, operand swizzles, the per-row Q quantizer, MFMA wrappers,
 // the per-block online softmax.
 #pragma once
-#include <type_traits>
-
 #include "sage_device.h"
 
 namespace sage {
@@ -49,74 +47,119 @@ struct QFrag {
   i32x8 f8[D / 64];
 };
 
-// Column of the c-th 8-element chunk a lane loads (c = 0 .. D/16 - 1), for lane half h.
-template <bool QK_INT8>
-__device__ __forceinline__ int qcol(int c, int h) {
-  return QK_INT8 ? 32 * (c >> 1) + 16 * h + 8 * (c & 1) : 64 * (c >> 2) + 32 * h + 8 * (c & 3);
+// The lane's number, formed anew (v_mbcnt): an epilogue that uses it does not keep the value from
+// the top of the kernel in a register across the main loop.
+__device__ __forceinline__ int lane_id() {
+  return (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
 }
 
-// Per-row Q quantization, shared by the main loop and the parity entry point.
-// sk1_t6i.hip:91-117 (int8) and sk1_t4a1s.hip:79-105 (fp8):
+// Bytes of LDS a wave needs to hand its quantized Q rows over (quant_q_tile): 32 rows x 64 columns.
+constexpr int Q_SCRATCH = 32 * 64;
+
+// Per-row quantization of a wave's 32 query rows q0 .. q0+31, shared by the main loops and the
+// parity entry point. sk1_t6i.hip:91-117 (int8) and sk1_t4a1s.hip:79-105 (fp8):
 //   amax = max(max_d |q|, 1e-12); qinv = RN(127/amax) (or 448); q8 = clamp(rne(RN(q*qinv)))
 //   (fp8: e4m3(clamp(RN(q*qinv), +-448))); sq = RN(amax/127) (or 448); c_q = RN(RN(sm*log2e)*sq).
-// Lanes q and q+32 hold the two halves of the row and exchange their partial absmax.
-// With `mu` (the plane's smooth_k mean, 128 fp32), also returns q . mu over the whole row in
-// `qmu` (fp32 products and sums, both lanes get it): the row's logsumexp correction for smooth_k.
+// The rows are loaded as they lie in memory, D/8 lanes of 16 bytes to a row (4 or 8 whole rows per
+// load), and a row's lanes share the work of its scale (row_max). The bytes reach the MFMA operand
+// layout (lane (q, h): row q, `qf`'s columns) through `scratch`, Q_SCRATCH bytes of LDS of the
+// wave's own, 64 columns at a time. What this replaces, each lane loading its own row and
+// quantizing it alone, touched 64 cache lines per load and took a wave 3.2k cycles of VALU issue:
+// with one 64-key block per query tile (768 tiles of 128 queries, three per CU) a call took
+// 16.8 us, of which 3.9 us per tile and CU were this and the epilogue.
+// `q`: the plane's row 0. Rows >= N are zero. sq, cq: of the lane's own row q0 + lane % 32.
+// With `mu` (the plane's smooth_k mean, D fp32), also q . mu of that row in `qmu` (fp32 products
+// and sums, in an order of its own): the row's logsumexp correction for smooth_k.
 template <typename T, bool QK_INT8, int D = HD>
-__device__ __forceinline__ void quant_q_row(const T* __restrict__ qrow_ptr, bool live, int h,
-                                            float sm_scale, QFrag<D>& qf, float& sq, float& cq,
-                                            const float* __restrict__ mu = nullptr,
-                                            float* qmu = nullptr) {
-  constexpr int NC = D / 16;   // 8-element chunks per lane (half a row)
-  float x[D / 2];
+__device__ __forceinline__ void quant_q_tile(const T* __restrict__ q, int q0, int N, int64_t q_sr,
+                                             int lane, float sm_scale, u8* scratch, QFrag<D>& qf,
+                                             float& sq, float& cq,
+                                             const float* __restrict__ mu = nullptr,
+                                             float* qmu = nullptr) {
+  constexpr int CG = D / 8, NR = CG / 2;   // lanes per row, rows per lane: 16, 8 or 8, 4
+  const int cg = lane % CG, rg = lane / CG, l32 = lane & 31, hh = lane >> 5;
+  const int own = (l32 / NR) * CG + l32 % NR;   // the lane that works out row l32's scale
+  const int row0 = q0 + NR * rg;
+  u32x4 w[NR];
+  const T* p = q + (int64_t)row0 * q_sr + 8 * cg;
 #pragma unroll
-  for (int c = 0; c < NC; ++c) {
-    const u32x4 w = live ? *(const u32x4*)(qrow_ptr + qcol<QK_INT8>(c, h)) : (u32x4){0u, 0u, 0u, 0u};
-    unpack8<T>(w, x + 8 * c);
+  for (int i = 0; i < NR; ++i)
+    w[i] = (row0 + i < N) ? *(const u32x4*)(p + i * q_sr) : (u32x4){0u, 0u, 0u, 0u};
+  float f[NR][8], m[NR];
+#pragma unroll
+  for (int i = 0; i < NR; ++i) {
+    unpack8<T>(w[i], f[i]);
+    m[i] = absmax8(f[i]);
   }
   if (mu) {
-    float d = 0.0f;
+    float v[8], sel = 0.0f;
+    const f32x4 m0 = *(const f32x4*)(mu + 8 * cg), m1 = *(const f32x4*)(mu + 8 * cg + 4);
 #pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      const f32x4 m0 = *(const f32x4*)(mu + qcol<QK_INT8>(c, h));
-      const f32x4 m1 = *(const f32x4*)(mu + qcol<QK_INT8>(c, h) + 4);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) d = __builtin_fmaf(x[8 * c + e], m0[e], d);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) d = __builtin_fmaf(x[8 * c + 4 + e], m1[e], d);
+    for (int e = 0; e < 4; ++e) {
+      v[e] = m0[e];
+      v[4 + e] = m1[e];
     }
-    *qmu = d + __shfl_xor(d, 32, 64);
-  }
-  float amax = 0.0f;
 #pragma unroll
-  for (int i = 0; i < D / 2; ++i) amax = fmaxf(amax, fabsf(x[i]));
-  amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
+    for (int i = 0; i < NR; ++i) {
+      float d = 0.0f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) d = __builtin_fmaf(f[i][e], v[e], d);
+#pragma unroll
+      for (int o = 1; o < CG; o <<= 1) d += __shfl_xor(d, o, 64);
+      sel = (lane & (NR - 1)) == i ? d : sel;
+    }
+    *qmu = __shfl(sel, own, 64);
+  }
+  float amax;
+  if constexpr (CG == 16)
+    amax = row_max<16>(m, cg);
+  else
+    amax = row_max(m, cg);
   amax = fmaxf(amax, SCALE_FLOOR);
   const float top = QK_INT8 ? I8_MAX : P_SCALE;
   const float qinv = __fdiv_rn(top, amax);
-  sq = __fdiv_rn(amax, top);
+  sq = __shfl(__fdiv_rn(amax, top), own, 64);
   const float smlog = sm_scale * LOG2E_F;
   cq = smlog * sq;
-  if (QK_INT8) {
+  u32x2 word[NR];
+  static_for<0, NR>([&](auto ic) {
+    constexpr int i = decltype(ic)::value;
+    const float y = group_bcast<CG, i>(qinv);
+    float z[8];
 #pragma unroll
-    for (int dd = 0; dd < D / 32; ++dd) {
-      const float* y = x + 16 * dd;
-      qf.i8[dd] = (i32x4){(int)i8x4(y[0] * qinv, y[1] * qinv, y[2] * qinv, y[3] * qinv),
-                          (int)i8x4(y[4] * qinv, y[5] * qinv, y[6] * qinv, y[7] * qinv),
-                          (int)i8x4(y[8] * qinv, y[9] * qinv, y[10] * qinv, y[11] * qinv),
-                          (int)i8x4(y[12] * qinv, y[13] * qinv, y[14] * qinv, y[15] * qinv)};
+    for (int e = 0; e < 8; ++e) {
+      z[e] = f[i][e] * y;
+      if (!QK_INT8) z[e] = fminf(fmaxf(z[e], -P_SCALE), P_SCALE);
     }
-  } else {
+    word[i] = QK_INT8 ? (u32x2){i8x4(z[0], z[1], z[2], z[3]), i8x4(z[4], z[5], z[6], z[7])}
+                      : (u32x2){fp8x4(z[0], z[1], z[2], z[3]), fp8x4(z[4], z[5], z[6], z[7])};
+  });
+  // scratch row r: 64 bytes, its 16-byte chunk c at position c ^ ((r >> 2) & 3), which keeps the
+  // operand reads (16 rows a pass) free of bank conflicts
 #pragma unroll
-    for (int dd = 0; dd < D / 64; ++dd) {
-      const float* y = x + 32 * dd;
-      float z[32];
+  for (int dd = 0; dd < D / 64; ++dd) {
+    const int c8 = cg - 8 * dd;              // this lane's 8-byte word of the 64 columns
+    if (c8 >= 0 && c8 < 8) {
 #pragma unroll
-      for (int i = 0; i < 32; ++i) z[i] = fminf(fmaxf(y[i] * qinv, -P_SCALE), P_SCALE);
-#pragma unroll
-      for (int k = 0; k < 8; ++k)
-        qf.f8[dd][k] = (int)fp8x4(z[4 * k], z[4 * k + 1], z[4 * k + 2], z[4 * k + 3]);
+      for (int i = 0; i < NR; ++i) {
+        const int r = NR * rg + i;
+        *(u32x2*)(scratch + 64 * r + 16 * ((c8 >> 1) ^ ((r >> 2) & 3)) + 8 * (c8 & 1)) = word[i];
+      }
     }
+    // the wave's own writes before its reads, and its reads before the next writes: LDS operations
+    // of a wave run in order; the fences keep the compiler from reordering them
+    asm volatile("" ::: "memory");
+    const u8* b = scratch + 64 * l32;
+    const int sw = (l32 >> 2) & 3;
+    if constexpr (QK_INT8) {
+      qf.i8[2 * dd] = *(const i32x4*)(b + 16 * (hh ^ sw));
+      qf.i8[2 * dd + 1] = *(const i32x4*)(b + 16 * ((2 + hh) ^ sw));
+    } else {
+      const i32x4 lo = *(const i32x4*)(b + 16 * ((2 * hh) ^ sw));
+      const i32x4 hi = *(const i32x4*)(b + 16 * ((2 * hh + 1) ^ sw));
+      qf.f8[dd] = (i32x8){lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+    }
+    asm volatile("" ::: "memory");
   }
 }
 
@@ -239,15 +282,6 @@ __device__ __forceinline__ float sum_halves(float v) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-
-// Calls f(integral_constant<int, i>) for i = I .. N-1, unrolled (compile-time lane selectors).
-template <int I, int N, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-  if constexpr (I < N) {
-    f(std::integral_constant<int, I>{});
-    static_for<I + 1, N>(f);
-  }
-}
 
 // Every lane receives lane n of its own 16-lane row (DPP row_newbcast:n). The compiler folds the
 // move into the consuming VALU instruction (v_mul_f32_dpp ... row_newbcast:n).
@@ -485,6 +519,70 @@ __device__ __forceinline__ void probs_tile(const f32x16 (&x)[2], float w, float 
     });
     pb[k4] = (int)fp8x4(p[0], p[1], p[2], p[3]);
   });
+}
+
+// Bytes of LDS a wave needs to write its output tile (store_o_tile): 32 rows x 64 columns of 2 bytes.
+constexpr int O_SCRATCH = 32 * 128;
+
+// The epilogue: rows q0 .. q0+31 of O = T(acc * inv) (with `vm`, the plane's V mean, T(fma(acc,
+// inv, vm[d]))), inv the lane's own row's factor. The accumulators hold one query per lane, so
+// storing them as they lie writes 16 bytes of each of 32 rows per instruction; they are turned in
+// `scratch` (O_SCRATCH bytes of LDS of the wave's own) 64 columns at a time and go out as whole
+// 128-byte row pieces, 8 rows per store.
+template <typename T, int D = HD>
+__device__ __forceinline__ void store_o_tile(const f32x16 (&acc)[D / 32], float inv,
+                                             const float* __restrict__ vm, T* __restrict__ o,
+                                             int q0, int N, int64_t o_sr, u8* scratch) {
+  const int lane = lane_id(), l32 = lane & 31, hh = lane >> 5;
+  // scratch row r: 128 bytes, its 16-byte chunk c at position c ^ ((r >> 1) & 7)
+  u8* const wr = scratch + 128 * l32 + 8 * hh;
+  const int wsw = (l32 >> 1) & 7;
+#pragma unroll
+  for (int dd = 0; dd < D / 64; ++dd) {
+    // x is rounded to fp32 before it is narrowed: left to itself the compiler forms some of the
+    // outputs with one rounding (v_fma_mixlo_f16), which ones depending on the surrounding code
+    auto put = [&](int t, int g, float (&x)[4]) {
+      T ov[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        asm("" : "+v"(x[e]));
+        ov[e] = (T)x[e];
+      }
+      u32x2 packed;
+      __builtin_memcpy(&packed, ov, 8);
+      *(u32x2*)(wr + 16 * ((4 * t + g) ^ wsw)) = packed;
+    };
+    if (vm) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const f32x4 m = *(const f32x4*)(vm + 64 * dd + 32 * t + 8 * g + 4 * hh);
+          float x[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) x[e] = __builtin_fmaf(acc[2 * dd + t][4 * g + e], inv, m[e]);
+          put(t, g, x);
+        }
+    } else {
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          float x[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) x[e] = acc[2 * dd + t][4 * g + e] * inv;
+          put(t, g, x);
+        }
+    }
+    asm volatile("" ::: "memory");   // the wave's own LDS writes, then its reads, in order
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int r = 8 * k + (lane >> 3), c = lane & 7;
+      const u32x4 x = *(const u32x4*)(scratch + 128 * r + 16 * (c ^ ((r >> 1) & 7)));
+      if (q0 + r < N) *(u32x4*)(o + (int64_t)(q0 + r) * o_sr + 64 * dd + 8 * c) = x;
+    }
+    asm volatile("" ::: "memory");
+  }
 }
 
 // The row's natural-log logsumexp of its scores times sm_scale, as the reference returns it

@@ -98,15 +98,12 @@ __global__ __launch_bounds__(AT) __attribute__((amdgpu_waves_per_eu(attn_waves(D
   //        logical chunk (l%4) ^ vswz(d).
   //   KC:  waves 0 and 1 carry floats 64w..64w+63 of the block's 128 (4 B/lane); waves 2 and 3
   //        repeat them into the tile's pad.
-  uint32_t k_off[NKV], v_off[NKV];
-#pragma unroll
-  for (int i = 0; i < NKV; ++i) {
-    const int I = NKV * w + i;
-    const int krow = (1024 / D) * I + lane / (D / 16), kpos = lane % (D / 16);
-    k_off[i] = (uint32_t)(krow * D + 16 * (kpos ^ kswz<D>(krow)));
-    const int d = 16 * I + (lane >> 2), vpos = lane & 3;
-    v_off[i] = (uint32_t)(d * Nk_pad + 16 * (vpos ^ vswz(d)));
-  }
+  // A wave's second request of a tile lies a whole number of swizzle periods on (8 or 16 rows of K,
+  // 16 of V^T), so it has the first one's per-lane offset from a base of its own.
+  const int krow = (1024 / D) * NKV * w + lane / (D / 16), kpos = lane % (D / 16);
+  const uint32_t k_off = (uint32_t)(krow * D + 16 * (kpos ^ kswz<D>(krow)));
+  const int vd = 16 * NKV * w + (lane >> 2), vpos = lane & 3;
+  const uint32_t v_off = (uint32_t)(vd * Nk_pad + 16 * (vpos ^ vswz(vd)));
   const uint32_t c_off = (uint32_t)(4 * (64 * (w & 1) + lane));
   const uint32_t c_dst = (uint32_t)(256 * w);
   auto dma = [&](int j, StageBuf<D>& buf) {
@@ -115,9 +112,9 @@ __global__ __launch_bounds__(AT) __attribute__((amdgpu_waves_per_eu(attn_waves(D
     const u8* cblk = (const u8*)KCb + (size_t)(128 * 4) * (uint32_t)j;
     const uint32_t kl = lds_addr(buf.k) + 1024 * NKV * w, vl = lds_addr(buf.v) + 1024 * NKV * w;
 #pragma unroll
-    for (int i = 0; i < NKV; ++i) dma16(kblk, k_off[i], kl + 1024 * i);
+    for (int i = 0; i < NKV; ++i) dma16(kblk + 1024 * i, k_off, kl + 1024 * i);
 #pragma unroll
-    for (int i = 0; i < NKV; ++i) dma16(vblk, v_off[i], vl + 1024 * i);
+    for (int i = 0; i < NKV; ++i) dma16(vblk + (size_t)(16 * i) * (uint32_t)Nk_pad, v_off, vl + 1024 * i);
     dma4(cblk, c_off, lds_addr(&buf.s) + c_dst);
   };
 
@@ -125,16 +122,16 @@ __global__ __launch_bounds__(AT) __attribute__((amdgpu_waves_per_eu(attn_waves(D
   dma(0, sB0);
   if (j_end > 1) dma(1, sB1);
 
-  // ---- Q: per-row quantization straight into MFMA fragments ----
+  // ---- Q: per-row quantization into MFMA fragments, through block 2's buffer ----
   QFrag<D> qf;
   float sq, cq;
   float qmu = 0.0f;   // q . mu for the logsumexp's smooth_k correction (when asked)
-  quant_q_row<T, QK_INT8, D>(Q + b * q_sb + hd * q_sh + (int64_t)qrow * q_sr, qrow < N, hh,
-                             sm_scale, qf, sq, cq,
-                             (LSE && KMEAN) ? KMEAN + (int64_t)kvp * D : nullptr, &qmu);
+  static_assert(4 * Q_SCRATCH <= sizeof(StageBuf<D>), "Q scratch");
+  quant_q_tile<T, QK_INT8, D>(Q + b * q_sb + hd * q_sh, q0, N, q_sr, lane, sm_scale,
+                              (u8*)&sB2 + Q_SCRATCH * w, qf, sq, cq,
+                              (LSE && KMEAN) ? KMEAN + (int64_t)kvp * D : nullptr, &qmu);
   (void)sq;
   if (LSE && hh == 0) s_qmu[32 * w + l32] = qmu;
-  const float Sb = Sfold[kvp];
 
   f32x16 acc[NDT];
 #pragma unroll
@@ -214,38 +211,15 @@ __global__ __launch_bounds__(AT) __attribute__((amdgpu_waves_per_eu(attn_waves(D
   mfma_result_fence();
 
   // ---------- epilogue: O = acc * S / (l * 448) (+ V's mean with smooth_v, one fma) ----------
-  // The row and lane half are formed again from the lane id (v_mbcnt), so that their values from
-  // the top of the kernel need not stay live across the loop.
-  const int lane_e = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
-  const int l32e = lane_e & 31, hhe = lane_e >> 5;
-  const int qrow_e = q0 + l32e;
-  if (qrow_e < N) {
-    if (LSE && hhe == 0)
-      LSE[(int64_t)bh * N + qrow_e] = row_lse(mc, l_i, sm_scale, s_qmu[32 * w + l32e]);
-    const float inv = (l_i > 0.0f) ? __fdiv_rn(Sb, l_i * P_SCALE) : 0.0f;
-    T* op = O + b * o_sb + hd * o_sh + (int64_t)qrow_e * o_sr;
-    const float* vmp = VMEAN ? VMEAN + (int64_t)kvp * D : nullptr;
-#pragma unroll
-    for (int dt = 0; dt < NDT; ++dt)
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int d = 32 * dt + 8 * g + 4 * hhe;
-        T ov[4];
-        if (vmp) {
-          const float4 vm = *(const float4*)(vmp + d);
-          ov[0] = (T)__builtin_fmaf(acc[dt][4 * g + 0], inv, vm.x);
-          ov[1] = (T)__builtin_fmaf(acc[dt][4 * g + 1], inv, vm.y);
-          ov[2] = (T)__builtin_fmaf(acc[dt][4 * g + 2], inv, vm.z);
-          ov[3] = (T)__builtin_fmaf(acc[dt][4 * g + 3], inv, vm.w);
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) ov[e] = (T)(acc[dt][4 * g + e] * inv);
-        }
-        uint2 packed;
-        __builtin_memcpy(&packed, ov, 8);
-        *(uint2*)(op + d) = packed;
-      }
-  }
+  // (every wave has passed the last block's barrier: the staging buffers are free)
+  static_assert(2 * O_SCRATCH <= sizeof(StageBuf<D>), "output scratch");
+  const int row = q0 + (lane_id() & 31);
+  if (LSE && lane_id() < 32 && row < N)
+    LSE[(int64_t)bh * N + row] = row_lse(mc, l_i, sm_scale, s_qmu[32 * w + (lane_id() & 31)]);
+  const float Sb = Sfold[kvp];
+  const float inv = (l_i > 0.0f) ? __fdiv_rn(Sb, l_i * P_SCALE) : 0.0f;
+  store_o_tile<T, D>(acc, inv, VMEAN ? VMEAN + (int64_t)kvp * D : nullptr, O + b * o_sb + hd * o_sh,
+                     q0, N, o_sr, (w < 2 ? (u8*)&sB0 : (u8*)&sB1) + O_SCRATCH * (w & 1));
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -261,11 +235,12 @@ __global__ __launch_bounds__(64) void quant_q_kernel(const T* __restrict__ Q, in
   const int nqb = (N + 31) / 32;
   const int bh = blockIdx.x / nqb, b = bh / H, hd = bh - b * H;
   const int lane = threadIdx.x, l32 = lane & 31, hh = lane >> 5;
-  const int qrow = (blockIdx.x - bh * nqb) * 32 + l32;
+  const int q0 = (blockIdx.x - bh * nqb) * 32, qrow = q0 + l32;
+  __shared__ __attribute__((aligned(16))) u8 scratch[Q_SCRATCH];
   QFrag<D> qf;
   float sq, cq;
-  quant_q_row<T, QK_INT8, D>(Q + b * q_sb + hd * q_sh + (int64_t)qrow * q_sr, qrow < N, hh,
-                             sm_scale, qf, sq, cq);
+  quant_q_tile<T, QK_INT8, D>(Q + b * q_sb + hd * q_sh, q0, N, q_sr, lane, sm_scale, scratch, qf,
+                              sq, cq);
   if (qrow >= N) return;
   u8* dst = Q8 + ((int64_t)bh * N + qrow) * D;
   if (QK_INT8) {

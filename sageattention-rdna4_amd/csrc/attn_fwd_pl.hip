@@ -80,6 +80,10 @@ __global__ __launch_bounds__(AT) __attribute__((amdgpu_waves_per_eu(pl_waves(D, 
   // block's LDS, 53248 bytes, is 26 units of 2 KB: three blocks fit a CU's 160 KB (one more
   // 2 KB unit each would leave room for two).
   __shared__ float xch[SPLIT ? 2 : 1][SPLIT ? 4 * 32 : 1];
+  // q . mu of each query row, for the logsumexp's smooth_k correction: parked here rather than in
+  // a register across the loop (SPLIT has the register, but no LDS to spare)
+  __shared__ float s_qmu[SPLIT ? 1 : BM];
+  __shared__ __attribute__((aligned(16))) u8 q_lds[D == 64 && !SPLIT ? 4 * Q_SCRATCH : 16];
   constexpr int NDT = D / 32;   // 32-channel output tiles per wave
   // 1 KB K and V^T requests per wave and block (each): a tile of D/16 KB over the 4 waves, or
   // over the 2 waves of a key group
@@ -124,39 +128,38 @@ __global__ __launch_bounds__(AT) __attribute__((amdgpu_waves_per_eu(pl_waves(D, 
 
   // ---- staging: per block every wave issues NKV KB of K and NKV KB of V^T; waves 0 and 1 also
   // 256 bytes of constants (SK, W). Layouts as in attn_fwd.hip.
-  uint32_t k_off[NKV], v_off[NKV];
-#pragma unroll
-  for (int i = 0; i < NKV; ++i) {
-    const int I = NKV * ws + i;
-    const int krow = (1024 / D) * I + lane / (D / 16), kpos = lane % (D / 16);
-    k_off[i] = (uint32_t)(krow * D + 16 * (kpos ^ kswz<D>(krow)));
-    const int d = 16 * I + (lane >> 2), vpos = lane & 3;
-    v_off[i] = (uint32_t)(d * Nk_pad + 16 * (vpos ^ vswz(d)));
-  }
+  // A wave's second request of a tile lies a whole number of swizzle periods on (8 or 16 rows of K,
+  // 16 of V^T), so it has the first one's per-lane offset from a base of its own.
+  const int krow = (1024 / D) * NKV * ws + lane / (D / 16), kpos = lane % (D / 16);
+  const uint32_t k_off = (uint32_t)(krow * D + 16 * (kpos ^ kswz<D>(krow)));
+  const int vd = 16 * NKV * ws + (lane >> 2), vpos = lane & 3;
+  const uint32_t v_off = (uint32_t)(vd * Nk_pad + 16 * (vpos ^ vswz(vd)));
   const uint32_t c_off = (uint32_t)(4 * lane);
   auto dma = [&](int j, PlBuf<D>& buf) {
     const u8* kblk = Kb + (size_t)(KS * BK * D) * (uint32_t)j;
     const u8* vblk = Vb + (size_t)(KS * BK) * (uint32_t)j;
     const uint32_t kl = lds_addr(buf.k) + 1024 * NKV * ws, vl = lds_addr(buf.v) + 1024 * NKV * ws;
 #pragma unroll
-    for (int i = 0; i < NKV; ++i) dma16(kblk, k_off[i], kl + 1024 * i);
+    for (int i = 0; i < NKV; ++i) dma16(kblk + 1024 * i, k_off, kl + 1024 * i);
 #pragma unroll
-    for (int i = 0; i < NKV; ++i) dma16(vblk, v_off[i], vl + 1024 * i);
+    for (int i = 0; i < NKV; ++i) dma16(vblk + (size_t)(16 * i) * (uint32_t)Nk_pad, v_off, vl + 1024 * i);
     if (ws < 2) dma4(Cb, c_off + c_blk * (uint32_t)j, lds_addr(ws == 0 ? buf.c.sk : buf.c.w));
   };
 
   if (!SPLIT || n_g > 0) dma(0, sB[0]);
   if ((SPLIT ? n_g : j_end) > 1) dma(1, sB[1]);
 
-  // ---- Q: per-row quantization straight into MFMA fragments ----
+  // ---- Q: per-row quantization into MFMA fragments, through the K tile of buffer 2 (head_dim 64
+  // without the split: an array of its own, that tile being too small for 4 waves) ----
+  u8* const q_scratch = (D == 64 && !SPLIT ? q_lds : sB[2].k) + Q_SCRATCH * ws;
   QFrag<D> qf;
   float sq, cq;
   float qmu = 0.0f;   // q . mu for the logsumexp's smooth_k correction (when asked)
-  quant_q_row<T, QK_INT8, D>(Q + b * q_sb + hd * q_sh + (int64_t)qrow * q_sr, qrow < N, hh,
-                             sm_scale, qf, sq, cq,
-                             (LSE && KMEAN) ? KMEAN + (int64_t)kvp * D : nullptr, &qmu);
+  quant_q_tile<T, QK_INT8, D>(Q + b * q_sb + hd * q_sh, q0, N, q_sr, lane, sm_scale,
+                              q_scratch, qf, sq, cq,
+                              (LSE && KMEAN) ? KMEAN + (int64_t)kvp * D : nullptr, &qmu);
   (void)sq;
-  const float Sb = Sfold[kvp];
+  if (!SPLIT && LSE && hh == 0) s_qmu[32 * w + l32] = qmu;
 
   f32x16 acc[NDT];
 #pragma unroll
@@ -233,9 +236,8 @@ __global__ __launch_bounds__(AT) __attribute__((amdgpu_waves_per_eu(pl_waves(D, 
     kw1 = buf.c.w[c + 16];
   };
   load_consts(sB[0]);
-  for (int j = 0; j <= j_end; ++j) {
+  for (int j = 0;; ++j) {   // ends at j == j_end, after that iteration's P.V
     const int pm = pc == 0 ? 2 : pc - 1, pn = pc == 2 ? 0 : pc + 1;
-    PlBuf<D>& bcur = sB[pc];
     PlBuf<D>& bprev = sB[pm];
     PlBuf<D>& bnext = sB[pn];
     const bool compute = j < w_end;
@@ -330,6 +332,9 @@ __global__ __launch_bounds__(AT) __attribute__((amdgpu_waves_per_eu(pl_waves(D, 
   for (int dt = 0; dt < NDT; ++dt) keep_live(acc[dt]);
   mfma_result_fence();
 
+  // Every wave is done with the staging ring: it becomes the waves' output scratch.
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  u8* o_scratch = (u8*)sBall + (SPLIT ? 64 * (16 * NDT + 2) * 4 : O_SCRATCH) * ws;
   if constexpr (SPLIT) {
     // Merge the key halves: group 1 parks O^T, mc and l of each lane in LDS (the staging ring is
     // free once every wave has passed the barrier), group 0 takes M = max(mc0, mc1) and
@@ -337,7 +342,6 @@ __global__ __launch_bounds__(AT) __attribute__((amdgpu_waves_per_eu(pl_waves(D, 
     // A half without keys has mc = -inf, so its factor is 0.
     constexpr int NE = 16 * NDT + 2;
     float* park = (float*)sBall + ws * (NE * 64);
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
     if (kg == 1) {
 #pragma unroll
       for (int dt = 0; dt < NDT; ++dt)
@@ -364,31 +368,14 @@ __global__ __launch_bounds__(AT) __attribute__((amdgpu_waves_per_eu(pl_waves(D, 
   }
 
   // ---------- epilogue: O = acc * S / (l * 448) (+ V's mean with smooth_v, one fma) ----------
-  if (qrow < N && kg == 0) {
-    if (LSE && hh == 0) LSE[(int64_t)bh * N + qrow] = row_lse(mc, l_i, sm_scale, qmu);
+  if (kg == 0) {
+    const int row = q0 + (lane_id() & 31);
+    if (LSE && lane_id() < 32 && row < N)
+      LSE[(int64_t)bh * N + row] = row_lse(mc, l_i, sm_scale, SPLIT ? qmu : s_qmu[32 * w + (lane_id() & 31)]);
+    const float Sb = Sfold[kvp];
     const float inv = (l_i > 0.0f) ? __fdiv_rn(Sb, l_i * P_SCALE) : 0.0f;
-    T* op = O + b * o_sb + hd * o_sh + (int64_t)qrow * o_sr;
-    const float* vmp = VMEAN ? VMEAN + (int64_t)kvp * D : nullptr;
-#pragma unroll
-    for (int dt = 0; dt < NDT; ++dt)
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int d = 32 * dt + 8 * g + 4 * hh;
-        T ov[4];
-        if (vmp) {
-          const float4 vm = *(const float4*)(vmp + d);
-          ov[0] = (T)__builtin_fmaf(acc[dt][4 * g + 0], inv, vm.x);
-          ov[1] = (T)__builtin_fmaf(acc[dt][4 * g + 1], inv, vm.y);
-          ov[2] = (T)__builtin_fmaf(acc[dt][4 * g + 2], inv, vm.z);
-          ov[3] = (T)__builtin_fmaf(acc[dt][4 * g + 3], inv, vm.w);
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) ov[e] = (T)(acc[dt][4 * g + e] * inv);
-        }
-        uint2 packed;
-        __builtin_memcpy(&packed, ov, 8);
-        *(uint2*)(op + d) = packed;
-      }
+    store_o_tile<T, D>(acc, inv, VMEAN ? VMEAN + (int64_t)kvp * D : nullptr,
+                       O + b * o_sb + hd * o_sh, q0, N, o_sr, o_scratch);
   }
 }
 

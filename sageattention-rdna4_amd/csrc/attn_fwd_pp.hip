@@ -101,14 +101,15 @@ __global__ __launch_bounds__(PP_T) __attribute__((amdgpu_waves_per_eu(2, 2))) vo
     dma_vc(1, 1);
   }
 
-  // ---- Q: per-row quantization straight into MFMA fragments ----
+  // ---- Q: per-row quantization into MFMA fragments, through block 2's buffer ----
   QFrag<HD> qf;
   float sq, cq;
   float qmu = 0.0f;   // q . mu for the logsumexp's smooth_k correction (when asked)
-  quant_q_row<T, QK_INT8>(Q + b * q_sb + hd * q_sh + (int64_t)qrow * q_sr, qrow < N, hh, sm_scale,
-                          qf, sq, cq, (LSE && KMEAN) ? KMEAN + (int64_t)kvp * HD : nullptr, &qmu);
+  static_assert(8 * Q_SCRATCH <= sizeof(StageBuf<HD>), "Q scratch");
+  quant_q_tile<T, QK_INT8>(Q + b * q_sb + hd * q_sh, q0, N, q_sr, lane, sm_scale,
+                           (u8*)&sB[2] + Q_SCRATCH * w, qf, sq, cq,
+                           (LSE && KMEAN) ? KMEAN + (int64_t)kvp * HD : nullptr, &qmu);
   (void)sq;
-  const float Sb = Sfold[kvp];
 
   f32x16 acc[4];
 #pragma unroll
@@ -303,32 +304,16 @@ __global__ __launch_bounds__(PP_T) __attribute__((amdgpu_waves_per_eu(2, 2))) vo
   mfma_result_fence();
 
   // ---------- epilogue: O = acc * S / (l * 448) (+ V's mean with smooth_v, one fma) ----------
-  if (qrow < N) {
-    if (LSE && hh == 0) LSE[(int64_t)bh * N + qrow] = row_lse(mc, l_i, sm_scale, qmu);
-    const float inv = (l_i > 0.0f) ? __fdiv_rn(Sb, l_i * P_SCALE) : 0.0f;
-    T* op = O + b * o_sb + hd * o_sh + (int64_t)qrow * o_sr;
-    const float* vmp = VMEAN ? VMEAN + (int64_t)kvp * HD : nullptr;
-#pragma unroll
-    for (int dt = 0; dt < 4; ++dt)
-#pragma unroll
-      for (int gg = 0; gg < 4; ++gg) {
-        const int d = 32 * dt + 8 * gg + 4 * hh;
-        T ov[4];
-        if (vmp) {
-          const float4 vm = *(const float4*)(vmp + d);
-          ov[0] = (T)__builtin_fmaf(acc[dt][4 * gg + 0], inv, vm.x);
-          ov[1] = (T)__builtin_fmaf(acc[dt][4 * gg + 1], inv, vm.y);
-          ov[2] = (T)__builtin_fmaf(acc[dt][4 * gg + 2], inv, vm.z);
-          ov[3] = (T)__builtin_fmaf(acc[dt][4 * gg + 3], inv, vm.w);
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) ov[e] = (T)(acc[dt][4 * gg + e] * inv);
-        }
-        uint2 packed;
-        __builtin_memcpy(&packed, ov, 8);
-        *(uint2*)(op + d) = packed;
-      }
-  }
+  // every wave is done with the staging ring: it becomes the waves' output scratch
+  static_assert(8 * O_SCRATCH <= sizeof(sB), "output scratch");
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  const int row = q0 + (lane_id() & 31);
+  if (LSE && lane_id() < 32 && row < N)
+    LSE[(int64_t)bh * N + row] = row_lse(mc, l_i, sm_scale, qmu);
+  const float Sb = Sfold[kvp];
+  const float inv = (l_i > 0.0f) ? __fdiv_rn(Sb, l_i * P_SCALE) : 0.0f;
+  store_o_tile<T>(acc, inv, VMEAN ? VMEAN + (int64_t)kvp * HD : nullptr, O + b * o_sb + hd * o_sh,
+                  q0, N, o_sr, (u8*)&sB[0] + O_SCRATCH * w);
 }
 
 template <typename T, bool QK_INT8, bool CAUSAL>

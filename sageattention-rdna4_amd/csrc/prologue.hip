@@ -32,8 +32,6 @@
 // N = 1024 21.7 / 16.0 us, N = 8771 99.4 / 80.4 us (436 MB moved, 5.4 TB/s), N = 47520 577 / 546 us;
 // 8 planes of 4096 21.1 / 11.5 us (its 96 mean partials were read one after another). A copy runs
 // at 5.1-5.6 TB/s on the same card and a read at 6.2 (7.0 with nontemporal loads).
-#include <type_traits>
-
 #include "sage_device.h"
 #include "sage_launch.h"
 
@@ -117,62 +115,6 @@ template <typename T>
 __device__ __forceinline__ void unpack_rows(const u32x4 (&w)[8], float (&f)[8][8]) {
 #pragma unroll
   for (int i = 0; i < 8; ++i) unpack8<T>(w[i], f[i]);
-}
-
-// max(m, |a|, |b|) as one v_max3_f32 (a plain fmaxf of inputs the compiler cannot prove quiet
-// costs a canonicalizing max per input). NaN inputs are ignored, as by fmaxf.
-__device__ __forceinline__ float max3abs(float m, float a, float b) {
-  float r;
-  asm("v_max3_f32 %0, %1, |%2|, |%3|" : "=v"(r) : "v"(m), "v"(a), "v"(b));
-  return r;
-}
-__device__ __forceinline__ float absmax8(const float* f) {
-  return max3abs(max3abs(max3abs(max3abs(0.0f, f[0], f[1]), f[2], f[3]), f[4], f[5]), f[6], f[7]);
-}
-// Non-negative floats order as their bits.
-__device__ __forceinline__ u32 umax(u32 a, u32 b) { return a > b ? a : b; }
-
-template <int CTRL>
-__device__ __forceinline__ u32 dpp_u32(u32 v) {
-  return (u32)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xF, 0xF, true);
-}
-
-// Eight values per lane, reduced over the aligned group of CG = 8 or 16 lanes that share the
-// rows: lane l of the group returns the group's maximum of value l & 7. Three exchange steps, each
-// of which hands over half of the values that are left (lanes 7 - l, l ^ 1, l ^ 2; and l ^ 8 for
-// 16 lanes): 22 operations, where a full reduction of each value takes 8 x 4 moves and maxima.
-template <int CG>
-__device__ __forceinline__ float row_max(const float (&m)[8], int lane) {
-  const bool b0 = lane & 1, b1 = lane & 2, b2 = lane & 4;
-  u32 a[4], c[2];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const u32 lo = __float_as_uint(m[j]), hi = __float_as_uint(m[j + 4]);
-    a[j] = umax(b2 ? hi : lo, dpp_u32<0x141>(b2 ? lo : hi));       // row_half_mirror
-  }
-#pragma unroll
-  for (int j = 0; j < 2; ++j)                                       // rows 2j, 2j + 1 (by b0)
-    c[j] = umax(b0 ? a[2 * j + 1] : a[2 * j], dpp_u32<0xB1>(b0 ? a[2 * j] : a[2 * j + 1]));
-  u32 r = umax(b1 ? c[1] : c[0], dpp_u32<0x4E>(b1 ? c[0] : c[1]));
-  if (CG == 16) r = umax(r, dpp_u32<0x128>(r));                     // row_ror:8
-  return __uint_as_float(r);
-}
-
-// Every lane of a CG-lane group receives lane I (0 .. 7) of its own group.
-template <int CG, int I>
-__device__ __forceinline__ float group_bcast(float v) {
-  int r = __builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + I, 0xF, 0xF, true);
-  if (CG == 8)   // two groups per 16-lane row: the second one's banks take its own lane
-    r = __builtin_amdgcn_update_dpp(r, __float_as_int(v), 0x158 + I, 0xF, 0xC, false);
-  return __int_as_float(r);
-}
-
-template <int I, int N, typename F>
-__device__ __forceinline__ void unroll_to(F&& f) {
-  if constexpr (I < N) {
-    f(std::integral_constant<int, I>{});
-    unroll_to<I + 1, N>(f);
-  }
 }
 
 // Two tokens' e4m3 bytes of one column into the low (HI = 0) or high half of a word.
@@ -355,7 +297,7 @@ __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(STATS_BLOCKS
       }
       // e4m3 bytes, two rows (tokens) at a time: col[e] holds tokens 0..3, 4..7 of column e
       u32 col[8][2];
-      unroll_to<0, 4>([&](auto ic) {
+      static_for<0, 4>([&](auto ic) {
         constexpr int i = 2 * decltype(ic)::value;
         const float s0 = group_bcast<CG, i>(sv), s1 = group_bcast<CG, i + 1>(sv);
         const float y0 = group_bcast<CG, i>(rsv), y1 = group_bcast<CG, i + 1>(rsv);
@@ -507,7 +449,7 @@ __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(QUANT_BLOCKS
     }
     // the quotients RN((k - mu) / sk) of each row, and their bytes
     u8* k8r = k8 + (int64_t)n * D;
-    unroll_to<0, 8>([&](auto ic) {
+    static_for<0, 8>([&](auto ic) {
       constexpr int i = decltype(ic)::value;
       const float s = group_bcast<CG, i>(sk), y = group_bcast<CG, i>(rsk);
       float x[8];

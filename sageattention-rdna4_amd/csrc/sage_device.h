@@ -11,6 +11,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 namespace sage {
 
 typedef uint8_t u8;
@@ -66,14 +68,17 @@ __device__ __forceinline__ uint32_t fp8x4(float a, float b, float c, float d) {
   return (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(c, d, r, true);
 }
 
-// Round half to even, clamp to [-128, 127], return the int8 byte.
-__device__ __forceinline__ uint32_t i8_rne(float x) {
-  const float r = fminf(fmaxf(__builtin_rintf(x), -128.0f), 127.0f);
-  return ((uint32_t)(int)r) & 0xffu;
-}
-// Four already-quantizable fp32 -> four int8 bytes (memory order a, b, c, d).
+// Four fp32, each rounded half to even and clamped to [-128, 127], as four int8 bytes (memory order
+// a, b, c, d). Adding 1.5 * 2^23 rounds the clamped value to an integer in the low mantissa bits,
+// whose low byte is the two's complement byte: per value a clamp and an add (about 4.3 and 2.3
+// cycles), where rounding, clamping, converting and masking take 19 cycles with their packing.
 __device__ __forceinline__ uint32_t i8x4(float a, float b, float c, float d) {
-  return i8_rne(a) | (i8_rne(b) << 8) | (i8_rne(c) << 16) | (i8_rne(d) << 24);
+  auto bits = [](float x) {
+    return __float_as_uint(__builtin_amdgcn_fmed3f(x, -128.0f, 127.0f) + 12582912.0f);
+  };
+  // v_perm_b32: selector bytes 0-3 take the second operand's bytes, 4-7 the first's, 12 is zero
+  return __builtin_amdgcn_perm(bits(b), bits(a), 0x0c0c0400u) |
+         __builtin_amdgcn_perm(bits(d), bits(c), 0x04000c0cu);
 }
 
 // RN(x / s) from y = RN(1 / s), in three operations instead of a full division: q = RN(x*y) is
@@ -105,6 +110,80 @@ __device__ __forceinline__ float maxg(float x) {
   x = fmaxf(x, dpp_mov<0x141>(x));   // row_half_mirror
   if (G == 16) x = fmaxf(x, dpp_mov<0x140>(x));   // row_mirror
   return x;
+}
+
+// max(m, |a|, |b|) as one v_max3_f32 (a plain fmaxf of inputs the compiler cannot prove quiet
+// costs a canonicalizing max per input). NaN inputs are ignored, as by fmaxf.
+__device__ __forceinline__ float max3abs(float m, float a, float b) {
+  float r;
+  asm("v_max3_f32 %0, %1, |%2|, |%3|" : "=v"(r) : "v"(m), "v"(a), "v"(b));
+  return r;
+}
+__device__ __forceinline__ float absmax8(const float* f) {
+  return max3abs(max3abs(max3abs(max3abs(0.0f, f[0], f[1]), f[2], f[3]), f[4], f[5]), f[6], f[7]);
+}
+// Non-negative floats order as their bits.
+__device__ __forceinline__ u32 umax(u32 a, u32 b) { return a > b ? a : b; }
+
+template <int CTRL>
+__device__ __forceinline__ u32 dpp_u32(u32 v) {
+  return (u32)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xF, 0xF, true);
+}
+
+// Calls f(integral_constant<int, i>) for i = I .. N-1, unrolled (compile-time lane selectors).
+template <int I, int N, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    static_for<I + 1, N>(f);
+  }
+}
+
+// Eight values per lane, reduced over the aligned group of CG = 8 or 16 lanes that share the
+// rows: lane l of the group returns the group's maximum of value l & 7. Three exchange steps, each
+// of which hands over half of the values that are left (lanes 7 - l, l ^ 1, l ^ 2; and l ^ 8 for
+// 16 lanes): 22 operations, where a full reduction of each value takes 8 x 4 moves and maxima.
+template <int CG>
+__device__ __forceinline__ float row_max(const float (&m)[8], int lane) {
+  const bool b0 = lane & 1, b1 = lane & 2, b2 = lane & 4;
+  u32 a[4], c[2];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const u32 lo = __float_as_uint(m[j]), hi = __float_as_uint(m[j + 4]);
+    a[j] = umax(b2 ? hi : lo, dpp_u32<0x141>(b2 ? lo : hi));       // row_half_mirror
+  }
+#pragma unroll
+  for (int j = 0; j < 2; ++j)                                       // rows 2j, 2j + 1 (by b0)
+    c[j] = umax(b0 ? a[2 * j + 1] : a[2 * j], dpp_u32<0xB1>(b0 ? a[2 * j] : a[2 * j + 1]));
+  u32 r = umax(b1 ? c[1] : c[0], dpp_u32<0x4E>(b1 ? c[0] : c[1]));
+  if (CG == 16) r = umax(r, dpp_u32<0x128>(r));                     // row_ror:8
+  return __uint_as_float(r);
+}
+
+// The same for four values per lane over a group of 8 lanes: lane l returns the maximum of value
+// l & 3 (lanes l ^ 1 and l ^ 2 exchange, then both quads).
+__device__ __forceinline__ float row_max(const float (&m)[4], int lane) {
+  const bool b0 = lane & 1, b1 = lane & 2;
+  u32 c[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const u32 lo = __float_as_uint(m[2 * j]), hi = __float_as_uint(m[2 * j + 1]);
+    c[j] = umax(b0 ? hi : lo, dpp_u32<0xB1>(b0 ? lo : hi));
+  }
+  const u32 r = umax(b1 ? c[1] : c[0], dpp_u32<0x4E>(b1 ? c[0] : c[1]));
+  // lane l ^ 4: row_shl:4 for the even quads, row_shr:4 for the odd ones
+  u32 o = (u32)__builtin_amdgcn_update_dpp(0, (int)r, 0x104, 0xF, 0x5, false);
+  o = (u32)__builtin_amdgcn_update_dpp((int)o, (int)r, 0x114, 0xF, 0xA, false);
+  return __uint_as_float(umax(r, o));
+}
+
+// Every lane of a CG-lane group receives lane I (0 .. 7) of its own group.
+template <int CG, int I>
+__device__ __forceinline__ float group_bcast(float v) {
+  int r = __builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + I, 0xF, 0xF, true);
+  if (CG == 8)   // two groups per 16-lane row: the second one's banks take its own lane
+    r = __builtin_amdgcn_update_dpp(r, __float_as_int(v), 0x158 + I, 0xF, 0xC, false);
+  return __int_as_float(r);
 }
 
 }  // namespace sage
