@@ -34,6 +34,7 @@
 // at the kernel: 64 queries per block, the key blocks shared out between two wave pairs.
 #include "attn_common.h"
 #include "sage_launch.h"
+#include "tile_order.h"
 
 namespace sage {
 
@@ -91,11 +92,17 @@ __global__ __launch_bounds__(AT) __attribute__((amdgpu_waves_per_eu(pl_waves(D, 
   constexpr int QB = SPLIT ? 64 : BM;          // queries per block
 
   // ---- which (plane, q-tile) this block runs: XCD-contiguous planes, longest causal tiles first
-  int id = blockIdx.x;
-  if (id < xcd_span) id = (id & 7) * (xcd_span >> 3) + (id >> 3);
-  const int bh = id / num_qt;
-  int qt = id - bh * num_qt;
-  if (CAUSAL) qt = num_qt - 1 - qt;
+  int bh, qt;
+  if (CAUSAL) {
+    const CausalTile t = causal_tile(blockIdx.x, xcd_span, num_qt, pl_waves(D, SPLIT));
+    bh = t.bh;
+    qt = num_qt - 1 - t.rank;
+  } else {
+    int id = blockIdx.x;
+    if (id < xcd_span) id = (id & 7) * (xcd_span >> 3) + (id >> 3);
+    bh = id / num_qt;
+    qt = id - bh * num_qt;
+  }
   const int b = bh / H, hd = bh - b * H;
   const int kvp = b * H_kv + hd / G;   // the K/V plane this query plane reads (GQA: G heads share it)
 

@@ -25,6 +25,7 @@
 // (needed in phase 2) and the V^T tile and constants of j+1 have landed.
 #include "attn_common.h"
 #include "sage_launch.h"
+#include "tile_order.h"
 
 namespace sage {
 
@@ -51,11 +52,17 @@ __global__ __launch_bounds__(PP_T) __attribute__((amdgpu_waves_per_eu(2, 2))) vo
   using I2 = std::integral_constant<int, 2>;
 
   // ---- which (plane, q-tile) this block runs: XCD-contiguous planes, longest causal tiles first
-  int id = blockIdx.x;
-  if (id < xcd_span) id = (id & 7) * (xcd_span >> 3) + (id >> 3);
-  const int bh = id / num_qt;
-  int qt = id - bh * num_qt;
-  if (CAUSAL) qt = num_qt - 1 - qt;
+  int bh, qt;
+  if (CAUSAL) {
+    const CausalTile t = causal_tile(blockIdx.x, xcd_span, num_qt, 1);
+    bh = t.bh;
+    qt = num_qt - 1 - t.rank;
+  } else {
+    int id = blockIdx.x;
+    if (id < xcd_span) id = (id & 7) * (xcd_span >> 3) + (id >> 3);
+    bh = id / num_qt;
+    qt = id - bh * num_qt;
+  }
   const int b = bh / H, hd = bh - b * H;
   const int kvp = b * H_kv + hd / G;   // the K/V plane this query plane reads (GQA: G heads share it)
 
