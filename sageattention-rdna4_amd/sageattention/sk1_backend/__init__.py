@@ -16,7 +16,6 @@ Mirrors `sageattention/sk1_backend/__init__.py` of the reference (`ENVELOPE` `:3
 call is outside the envelope or (with `strict=False`) when the library fails.
 """
 import sys
-from contextlib import nullcontext
 
 import torch
 
@@ -46,6 +45,8 @@ ENVELOPE = dict(
 )
 
 _LOGGED = set()
+#: device index -> architecture, which a process's device keeps
+_ARCHS = {}
 
 
 def _log_once(msg):
@@ -61,10 +62,14 @@ def device_arch(device=None) -> str:
     (`sageattention/sk1_backend/__init__.py:393-410` of the reference).
     """
     try:
-        if device is None:
-            device = torch.cuda.current_device()
-        name = getattr(torch.cuda.get_device_properties(device), "gcnArchName", "") or ""
-        return name.split(":", 1)[0]
+        index = device.index if isinstance(device, torch.device) else device
+        if index is None:
+            index = torch.cuda.current_device()
+        arch = _ARCHS.get(index)
+        if arch is None:
+            name = getattr(torch.cuda.get_device_properties(index), "gcnArchName", "") or ""
+            arch = _ARCHS[index] = name.split(":", 1)[0]
+        return arch
     except Exception:  # noqa: BLE001
         return ""
 
@@ -185,8 +190,8 @@ def sk1_forward(lib, q, k, v, *, tensor_layout="HND", is_causal=False, sm_scale=
         qq, kk, vv = q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2)
     else:
         qq, kk, vv = q, k, v
-    B, H, N, D = (int(x) for x in qq.shape)
-    H_kv, N_kv = int(kk.shape[1]), int(kk.shape[2])
+    B, H, N, D = qq.shape
+    _, H_kv, N_kv, _ = kk.shape
     BH_kv = B * H_kv
     is_bf16 = q.dtype == torch.bfloat16
     qk_int8 = (not is_bf16) and (int8 is None or bool(int8))
@@ -196,18 +201,20 @@ def sk1_forward(lib, q, k, v, *, tensor_layout="HND", is_causal=False, sm_scale=
     # Every temporary of the call in one allocation, 256-byte aligned parts: the prologue's
     # outputs per K/V plane (B*H_kv planes of N_kv keys) -- K8, SK, V8T, SV, S, KCONST -- its
     # workspace, and K's mean (for the logsumexp) and V's mean (smooth_v) when used.
-    el8, nf = BH_kv * n_pad * D, BH_kv * n_pad * 4
+    el8, nf = BH_kv * n_pad * D, BH_kv * n_pad * 4     # n_pad is a multiple of 64: both are of 256
     ws_bytes = lib.workspace_bytes(BH_kv, N_kv)
-    parts = [("k8", el8), ("sk", nf), ("v8t", el8), ("sv", nf), ("s", BH_kv * 4),
-             ("kconst", 2 * nf), ("ws", ws_bytes)]
+    s_off = 2 * (el8 + nf)
+    kc_off = s_off + (BH_kv * 4 + 255) // 256 * 256
+    ws_off = kc_off + 2 * nf
+    off = {"k8": 0, "sk": el8, "v8t": el8 + nf, "sv": 2 * el8 + nf, "s": s_off, "kconst": kc_off,
+           "ws": ws_off}
+    total = ws_off + (ws_bytes + 255) // 256 * 256
     if return_lse and smooth_k:
-        parts.append(("kmean", BH_kv * D * 4))
+        off["kmean"] = total
+        total += (BH_kv * D * 4 + 255) // 256 * 256
     if smooth_v:
-        parts.append(("vmean", BH_kv * D * 4))
-    off, total = {}, 0
-    for name, nbytes in parts:
-        off[name] = total
-        total += (nbytes + 255) // 256 * 256
+        off["vmean"] = total
+        total += (BH_kv * D * 4 + 255) // 256 * 256
     tmp = torch.empty(total, device=dev, dtype=torch.uint8)
     lse = torch.empty(B, H, N, device=dev, dtype=torch.float32) if return_lse else None
     if tensor_layout == "NHD":
@@ -216,10 +223,14 @@ def sk1_forward(lib, q, k, v, *, tensor_layout="HND", is_causal=False, sm_scale=
     else:
         out = torch.empty(B, H, N, D, device=dev, dtype=q.dtype)
         oo = out
-    ctx = torch.cuda.device(dev) if dev.index != torch.cuda.current_device() else nullcontext()
-    with ctx:
+    def launch():
         lib.prologue_and_main(qq, kk, vv, oo, tmp.data_ptr(), off, ws_bytes, n_pad,
                               qk_int8=qk_int8, smooth_k=bool(smooth_k), smooth_v=bool(smooth_v),
                               causal=bool(is_causal), sm_scale=sm, kernel=kernel, lse=lse,
                               stream=torch_stream(dev), events=events)
+    if dev.index == torch.cuda.current_device():
+        launch()
+    else:
+        with torch.cuda.device(dev):
+            launch()
     return (out, lse) if return_lse else out

@@ -12,6 +12,7 @@ vocabulary `REFUSALS`, `check`, `quant_kv` (returns `(k8, sk, v8t, sv)` freshly 
 * `floor` is fixed at the reference's 1e-12.
 """
 import collections
+from contextlib import nullcontext
 
 import torch
 
@@ -117,7 +118,8 @@ class HipPrologue:
             s = torch.empty(BH, device=dev, dtype=torch.float32)
             mean = torch.empty(BH, D, device=dev, dtype=torch.float32) if smooth_k else None
             ws = torch.empty(self.lib.workspace_bytes(BH, N), device=dev, dtype=torch.uint8)
-            with torch.cuda.device(dev):
+            on_dev = dev.index == torch.cuda.current_device()
+            with nullcontext() if on_dev else torch.cuda.device(dev):
                 self.lib.kv_prologue(k, v, k8, sk, v8t, sv, s, mean, ws, k_int8=int8,
                                      smooth_k=smooth_k, fold=fold, n_pad=n_pad)
         except Exception as e:  # noqa: BLE001 - the reference's prologue contract is "never raises"

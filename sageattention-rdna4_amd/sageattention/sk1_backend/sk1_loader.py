@@ -51,10 +51,17 @@ def strided_view_reason(t, name="t"):
     st = [int(s) for s in st]
     if any(s <= 0 for s in st):
         return "stride_nonpos"
-    if any(st[i] % 8 for i in (0, 1, 2)):
+    if (st[0] | st[1] | st[2]) & 7:
         return "stride_align"
-    if int(t.data_ptr()) % 16:
+    if int(t.data_ptr()) & 15:
         return "ptr_align"
+    n, d = t.shape, t.shape[3]
+    # batches of rows of heads (NHD, fused-QKV views) or of heads of rows (HND slices), each level
+    # at least the extent of the one below: injective, the usual case
+    if st[0] >= st[2] * n[2] and st[2] >= st[1] * n[1] and st[1] >= d:
+        return None
+    if st[0] >= st[1] * n[1] and st[1] >= st[2] * n[2] and st[2] >= d:
+        return None
     dims = sorted((st[i], int(t.shape[i])) for i in range(4) if int(t.shape[i]) > 1)
     for (s0, n0), (s1, _) in zip(dims, dims[1:]):
         if s1 < s0 * n0:
@@ -62,7 +69,14 @@ def strided_view_reason(t, name="t"):
     return None
 
 
+#: the current stream's handle by device index, without a torch.cuda.Stream object around it
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def torch_stream(device=None):
+    index = device.index if isinstance(device, torch.device) else None
+    if index is not None and _raw_stream is not None:
+        return _raw_stream(index)
     return int(torch.cuda.current_stream(device).cuda_stream)
 
 
@@ -185,15 +199,15 @@ class SageLib:
         `sage_kv_prologue`).
         `kconst` (optional) receives the main loop's per-key constants, (B*H, N_pad/64, 2, 64);
         with `smooth_v`, `vmean` ((B*H, 128) fp32) receives V's sequence mean."""
-        B, H, N, D = (int(x) for x in k.shape)
+        B, H, N, D = k.shape
+        k_sb, k_sh, k_sr, _ = k.stride()
+        v_sb, v_sh, v_sr, _ = v.stride()
         rc = self.lib.sage_kv_prologue(
             _dtype_code(k.dtype), int(bool(k_int8)), int(bool(smooth_k)), int(bool(smooth_v)),
-            int(bool(fold)), _ptr(k), k.stride(0), k.stride(1), k.stride(2),
-            _ptr(v), v.stride(0), v.stride(1), v.stride(2),
-            B, H, N, int(n_pad), D, _ptr(k8), _ptr(sk), _ptr(v8t), _ptr(sv), _ptr(mean),
-            _ptr(vmean), _ptr(s), _ptr(kconst), _ptr(workspace),
-            int(workspace.numel() * workspace.element_size()),
-            ctypes.c_void_p(torch_stream(k.device)))
+            int(bool(fold)), k.data_ptr(), k_sb, k_sh, k_sr, v.data_ptr(), v_sb, v_sh, v_sr,
+            B, H, N, int(n_pad), D, k8.data_ptr(), sk.data_ptr(), v8t.data_ptr(), sv.data_ptr(),
+            _ptr(mean), _ptr(vmean), s.data_ptr(), _ptr(kconst), workspace.data_ptr(),
+            workspace.numel() * workspace.element_size(), torch_stream(k.device))
         self._check(rc, "sage_kv_prologue")
 
     def prologue_and_main(self, q, k, v, o, base, off, ws_bytes, n_pad, *, qk_int8, smooth_k,
@@ -204,32 +218,35 @@ class SageLib:
         `q`, `o` are logical (B, H, N, D) views, `k`, `v` (B, H_kv, N_kv, D). One stream handle for
         both calls; `events` (three, optional) are recorded before, between and after them."""
         B, H, N, D = q.shape
-        H_kv, N_kv = k.shape[1], k.shape[2]
-        vp = ctypes.c_void_p
-
-        def at(name):
-            o_ = off.get(name)
-            return None if o_ is None else vp(base + o_)
-
+        _, H_kv, N_kv, _ = k.shape
+        # addresses go as plain ints (None: a null pointer), which ctypes converts by the argtypes
+        k8, v8t, s = base + off["k8"], base + off["v8t"], base + off["s"]
+        kconst = base + off["kconst"]
+        kmean, vmean = off.get("kmean"), off.get("vmean")
+        kmean = None if kmean is None else base + kmean
+        vmean = None if vmean is None else base + vmean
         dt = _dtype_code(q.dtype)
-        st = vp(stream)
-        ks, vs, qs, os_ = k.stride(), v.stride(), q.stride(), o.stride()
+        int8 = int(qk_int8)
+        k_sb, k_sh, k_sr, _ = k.stride()
+        v_sb, v_sh, v_sr, _ = v.stride()
+        q_sb, q_sh, q_sr, _ = q.stride()
+        o_sb, o_sh, o_sr, _ = o.stride()
         if events is not None:
             events[0].record()
         rc = self.lib.sage_kv_prologue(
-            dt, int(qk_int8), int(smooth_k), int(smooth_v), 1, vp(k.data_ptr()), ks[0], ks[1],
-            ks[2], vp(v.data_ptr()), vs[0], vs[1], vs[2], B, H_kv, N_kv, n_pad, D, at("k8"),
-            at("sk"), at("v8t"), at("sv"), at("kmean"), at("vmean"), at("s"), at("kconst"),
-            at("ws"), ws_bytes, st)
-        self._check(rc, "sage_kv_prologue")
+            dt, int8, int(smooth_k), int(smooth_v), 1, k.data_ptr(), k_sb, k_sh, k_sr,
+            v.data_ptr(), v_sb, v_sh, v_sr, B, H_kv, N_kv, n_pad, D, k8, base + off["sk"], v8t,
+            base + off["sv"], kmean, vmean, s, kconst, base + off["ws"], ws_bytes, stream)
+        if rc:
+            self._check(rc, "sage_kv_prologue")
         if events is not None:
             events[1].record()
         rc = self.lib.sage_attn_fwd_ex(
-            dt, int(qk_int8), int(causal), vp(q.data_ptr()), qs[0], qs[1], qs[2], at("k8"),
-            at("kconst"), at("v8t"), at("s"), vp(o.data_ptr()), os_[0], os_[1], os_[2], B, H, N,
-            H_kv, N_kv, n_pad, D, ctypes.c_float(sm_scale), int(kernel), _ptr(lse), at("kmean"),
-            at("vmean"), st)
-        self._check(rc, "sage_attn_fwd")
+            dt, int8, int(causal), q.data_ptr(), q_sb, q_sh, q_sr, k8, kconst, v8t, s,
+            o.data_ptr(), o_sb, o_sh, o_sr, B, H, N, H_kv, N_kv, n_pad, D, sm_scale, int(kernel),
+            None if lse is None else lse.data_ptr(), kmean, vmean, stream)
+        if rc:
+            self._check(rc, "sage_attn_fwd")
         if events is not None:
             events[2].record()
 
