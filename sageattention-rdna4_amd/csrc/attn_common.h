@@ -317,14 +317,22 @@ struct BlockShift {
 
 // block_max: the first part of scores_block -- x = fp32(Q8.K8) * SK over the raw scores, masked
 // keys -inf -- returning this lane's query's max over the block's 64 keys.
-template <bool QK_INT8, bool CAUSAL, int NCONV = 0>
+// With SK4 the scales are sk4's (the lane half's 32 SK values, in LDS or in registers) instead of
+// DPP broadcasts of sk0 and sk1.
+template <bool QK_INT8, bool CAUSAL, int NCONV = 0, bool SK4 = false>
 __device__ __forceinline__ float block_max(f32x16 (&sx)[2], float sk0, float sk1, int j, int q0,
-                                           int qrow, int N, int hh) {
+                                           int qrow, int N, int hh, const f32x4* sk4 = nullptr) {
+  f32x4 s4;
   static_for<0, 32>([&](auto ic) {
     constexpr int jj = decltype(ic)::value;
     const float v = sx[jj >> 4][jj & 15];
     const float d = (QK_INT8 && jj >= NCONV) ? (float)__float_as_int(v) : v;
-    sx[jj >> 4][jj & 15] = d * row_bcast<jj & 15>(jj < 16 ? sk0 : sk1);
+    if constexpr (SK4) {
+      if constexpr ((jj & 3) == 0) s4 = sk4[jj >> 2];
+      sx[jj >> 4][jj & 15] = d * s4[jj & 3];
+    } else {
+      sx[jj >> 4][jj & 15] = d * row_bcast<jj & 15>(jj < 16 ? sk0 : sk1);
+    }
   });
   const bool need_mask = CAUSAL ? (BK * j + BK - 1 > q0) : (BK * j + BK > N);
   if (need_mask) {
@@ -359,11 +367,12 @@ __device__ __forceinline__ float shift_of(float m, float cq) {
   return mc;
 }
 
-template <bool QK_INT8, bool CAUSAL, int NCONV = 0>
+template <bool QK_INT8, bool CAUSAL, int NCONV = 0, bool SK4 = false>
 __device__ __forceinline__ BlockShift scores_block(f32x16 (&sx)[2], float sk0, float sk1, int j, int q0,
                                                    int qrow, int N, int hh, float cq, float& m_x,
-                                                   float& mc) {
-  const float mx = block_max<QK_INT8, CAUSAL, NCONV>(sx, sk0, sk1, j, q0, qrow, N, hh);
+                                                   float& mc, const f32x4* sk4 = nullptr) {
+  const float mx =
+      block_max<QK_INT8, CAUSAL, NCONV, SK4>(sx, sk0, sk1, j, q0, qrow, N, hh, sk4);
   const float m_new = fmaxf(m_x, mx);
   const float mc_new = shift_of(m_new, cq);
   const float alpha = (m_new != m_x) ? __builtin_amdgcn_exp2f(mc - mc_new) : 1.0f;
@@ -499,23 +508,27 @@ __device__ __forceinline__ f32x16 qk_tile(const u8* __restrict__ kbuf, const QFr
 
 // The exponentials, row-sum partials and e4m3 P of the 16 scores of tile T (keys 32h + 16T + r):
 // the same operations, in the same order per score and per partial sum, as probs_block
-// (attn_common.h), which does both tiles in one pass. w: the tile's W broadcast source.
-template <int T>
+// (attn_common.h), which does both tiles in one pass. w: the tile's W broadcast source; with W4
+// w4 holds the lane half's 32 values instead (in LDS or in registers).
+template <int T, bool W4 = false>
 __device__ __forceinline__ void probs_tile(const f32x16 (&x)[2], float w, float cq, float mc,
-                                           float (&ps)[4], i32x8& pb) {
+                                           float (&ps)[4], i32x8& pb,
+                                           const f32x4* w4 = nullptr) {
   // W enters through an opaque copy: otherwise its broadcasts can be hoisted away from the
   // multiplies they fold into (one extra move, and a live register, per score)
   asm volatile("" : "+v"(w));
   static_for<0, 4>([&](auto k4c) {
     constexpr int k4 = decltype(k4c)::value + 4 * T;
     float p[4];
+    f32x4 wk;
+    if constexpr (W4) wk = w4[k4];
     static_for<0, 4>([&](auto ec) {
       constexpr int e = decltype(ec)::value;
       constexpr int jj = 4 * k4 + e;
       p[e] = __builtin_amdgcn_fmed3f(__builtin_amdgcn_exp2f(__builtin_fmaf(x[T][jj & 15], cq, -mc)),
                                      0.0f, 1.0f);
       ps[e] = k4 ? ps[e] + p[e] : p[e];
-      p[e] *= row_bcast<jj & 15>(w);
+      p[e] *= W4 ? wk[e] : row_bcast<jj & 15>(w);
     });
     pb[k4] = (int)fp8x4(p[0], p[1], p[2], p[3]);
   });

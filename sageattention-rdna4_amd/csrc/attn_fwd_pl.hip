@@ -21,7 +21,7 @@
 // SIMD, which belong to other blocks and drift freely against it.
 //
 // Block: 4 waves x 32 queries (128 queries of one plane), one wave per SIMD; three blocks per CU
-// at head_dim 128 (168 VGPRs, 3 x 50 KB LDS), four at head_dim 64. K tiles, V^T tiles and the
+// at head_dim 128 (168 VGPRs, 3 x 50 KB LDS), four at head_dim 64 (128 VGPRs, 34 KB). K tiles, V^T tiles and the
 // per-key constants go global -> LDS directly (global_load_lds) into a ring of three buffers: the
 // tiles of block j+2 are requested in iteration j, after the iteration's barrier, into the buffer
 // block j-1 used (whose V^T tile every wave read before that barrier).
@@ -66,7 +66,7 @@ constexpr int pl_waves(int D, bool split = false) { return split ? 3 : (D == 64 
 // sum and O^T relative to its last shift; at the end group 1 hands them to group 0 through LDS,
 // which rescales both to the larger shift and writes the output. Only the fp32 sums differ from
 // the sequential loop's (rescaled per group, then merged): rounding-level output differences.
-template <typename T, bool QK_INT8, bool CAUSAL, int D, bool SPLIT = false>
+template <typename T, bool QK_INT8, bool CAUSAL, int D, bool SPLIT = false, bool CLDS = false>
 __global__ __launch_bounds__(AT) __attribute__((amdgpu_waves_per_eu(pl_waves(D, SPLIT), pl_waves(D, SPLIT)))) void attn_fwd_pl_kernel(
     const T* __restrict__ Q, const u8* __restrict__ K8, const float* __restrict__ SKr,
     int64_t sk_plane, int64_t sk_block, const float* __restrict__ Wr, int64_t w_plane,
@@ -234,7 +234,7 @@ __global__ __launch_bounds__(AT) __attribute__((amdgpu_waves_per_eu(pl_waves(D, 
   // copy can read an MFMA result before the MFMA has written it.
   int pc = 0;   // j % 3
   // block j's per-key constants, read from LDS one iteration ahead (block 0's here)
-  float ksk0, ksk1, kw0, kw1;
+  float ksk0 = 0.0f, ksk1 = 0.0f, kw0 = 0.0f, kw1 = 0.0f;
   auto load_consts = [&](const PlBuf<D>& buf) {
     const int c = 32 * hh + (lane & 15);
     ksk0 = buf.c.sk[c];
@@ -242,12 +242,14 @@ __global__ __launch_bounds__(AT) __attribute__((amdgpu_waves_per_eu(pl_waves(D, 
     kw0 = buf.c.w[c];
     kw1 = buf.c.w[c + 16];
   };
-  load_consts(sB[0]);
+  if constexpr (!CLDS) load_consts(sB[0]);
   for (int j = 0;; ++j) {   // ends at j == j_end, after that iteration's P.V
     const int pm = pc == 0 ? 2 : pc - 1, pn = pc == 2 ? 0 : pc + 1;
     PlBuf<D>& bprev = sB[pm];
     PlBuf<D>& bnext = sB[pn];
     const bool compute = j < w_end;
+    const f32x4* sk4 = (const f32x4*)(sB[pc].c.sk + 32 * hh);
+    const f32x4* w4 = (const f32x4*)(sB[pc].c.w + 32 * hh);
     // Each section is a scheduling region of its own: the compiler neither hoists one
     // iteration's LDS operand reads into the previous one nor mixes the sections' live ranges.
     __builtin_amdgcn_sched_barrier(0);
@@ -268,9 +270,11 @@ __global__ __launch_bounds__(AT) __attribute__((amdgpu_waves_per_eu(pl_waves(D, 
       w0 = kw0 * w_mul;
       w1 = kw1 * w_mul;
       if constexpr (SPLIT) {
-        mx = block_max<QK_INT8, false>(st, ksk0, ksk1, KS * j + kg, q0, qrow, Nk, hh);
+        mx = block_max<QK_INT8, false, 0, CLDS>(st, ksk0, ksk1, KS * j + kg, q0, qrow, Nk, hh,
+                                                sk4);
       } else {
-        sh = scores_block<QK_INT8, CAUSAL>(st, ksk0, ksk1, j, q0, qrow, Nk, hh, cq, m_x, mc);
+        sh = scores_block<QK_INT8, CAUSAL, 0, CLDS>(st, ksk0, ksk1, j, q0, qrow, Nk, hh, cq, m_x,
+                                                    mc, sk4);
         // acc *= alpha before block j's P.V (issued next iteration); P.V of block j-1 was
         // issued above, a whole scores pass ago
         rescale_acc(acc, sh.alpha);
@@ -317,11 +321,11 @@ __global__ __launch_bounds__(AT) __attribute__((amdgpu_waves_per_eu(pl_waves(D, 
     // of tile t as soon as they are consumed
     if (compute) {
       float ps[4];
-      probs_tile<0>(st, w0, cq, sh.mc, ps, pb);
+      probs_tile<0, CLDS>(st, w0, cq, sh.mc, ps, pb, w4);
       st[0] = qk_tile<QK_INT8, D>(bnext.k, qf, krow0, ksw0, hh);
       keep_live(st[0]);
       __builtin_amdgcn_sched_barrier(0);
-      probs_tile<1>(st, w1, cq, sh.mc, ps, pb);
+      probs_tile<1, CLDS>(st, w1, cq, sh.mc, ps, pb, w4);
       st[1] = qk_tile<QK_INT8, D>(bnext.k, qf, krow1, ksw1, hh);
       keep_live(st[1]);
       asm volatile("" ::"v"(pb));
@@ -329,7 +333,7 @@ __global__ __launch_bounds__(AT) __attribute__((amdgpu_waves_per_eu(pl_waves(D, 
       const float psum = sum_halves((ps[0] + ps[1]) + (ps[2] + ps[3]));
       l_i = __builtin_fmaf(l_i, sh.alpha, psum);
       // block j+1's constants: in buffer (j+1) % 3 since this iteration's barrier
-      load_consts(bnext);
+      if constexpr (!CLDS) load_consts(bnext);
     }
     pc = pn;
   }
@@ -386,7 +390,7 @@ __global__ __launch_bounds__(AT) __attribute__((amdgpu_waves_per_eu(pl_waves(D, 
   }
 }
 
-template <typename T, bool QK_INT8, bool CAUSAL, int D, bool SPLIT = false>
+template <typename T, bool QK_INT8, bool CAUSAL, int D, bool SPLIT = false, bool CLDS = false>
 static void launch_pl_d(const AttnArgs& a, hipStream_t stream) {
   const int BH = (int)(a.B * a.H);
   const int num_qt = (int)((a.N + (SPLIT ? 64 : BM) - 1) / (SPLIT ? 64 : BM));
@@ -397,7 +401,8 @@ static void launch_pl_d(const AttnArgs& a, hipStream_t stream) {
   const float* skr = kc ? a.kconst : a.sk;
   const float* wr = kc ? a.kconst + BK : a.svp;
   const int64_t plane = kc ? 2 * a.N_kv_pad : a.N_kv_pad, blk = kc ? 2 * BK : BK;
-  hipLaunchKernelGGL((attn_fwd_pl_kernel<T, QK_INT8, CAUSAL, D, SPLIT>), dim3(total), dim3(AT), 0, stream,
+  hipLaunchKernelGGL((attn_fwd_pl_kernel<T, QK_INT8, CAUSAL, D, SPLIT, CLDS>), dim3(total),
+                     dim3(AT), 0, stream,
                      (const T*)a.q, (const u8*)a.k8, skr, plane, blk, wr, plane, blk,
                      kc ? 1.0f : P_SCALE, (const u8*)a.v8t, a.s, (T*)a.o, a.q_sb, a.q_sh, a.q_sr,
                      a.o_sb, a.o_sh, a.o_sr, (int)a.H, (int)a.H_kv, (int)(a.H / a.H_kv), (int)a.N,
@@ -405,17 +410,36 @@ static void launch_pl_d(const AttnArgs& a, hipStream_t stream) {
                      a.vmean);
 }
 
+// Where a head_dim 64 softmax takes its per-key constants from (CLDS; same values, same bits). As
+// DPP broadcasts they cost a 4-cycle multiply per score instead of a 2-cycle one; as 16-byte LDS
+// reads that a half-wave shares they cost the read's latency, which only other waves of the SIMD
+// hide. So LDS once a launch keeps several blocks on every CU: main loop, DPP -> LDS, at 1 block
+// per CU 62.7 -> 69.3 us, at 2 92.4 -> 93.1, at 2.5 128.0 -> 123.8, at 4 155.7 -> 153.0
+// (N = 4096), 30 planes of 17550 2591 -> 2514; on a card that throttled under its power cap 6 planes
+// of 32768 went 1809 -> 1836 (1765 -> 1738 on one that did not). A causal launch of fewer than ~3 ends in its longest tiles, each alone on its SIMDs:
+// at 3 63.8 -> 71.3, at 3.5 89.7 -> 84.4, at 4 89.0 -> 85.1. The key split's blocks: at 1
+// 39.3 -> 42.1, at 1.25 18.0 -> 17.8, at 2.5 72.7 -> 69.6. head_dim 128 (three blocks per CU,
+// twice the matrix work a score) gained nothing.
+static bool consts_from_lds(int64_t blocks, bool causal, bool split) {
+  return blocks > 8 * XCD_CUS * (split ? 1 : causal ? 3 : 2);
+}
+
 template <typename T, bool QK_INT8, bool CAUSAL>
 static void launch_pl_t(const AttnArgs& a, hipStream_t stream) {
-  if (a.D == 64)
-    launch_pl_d<T, QK_INT8, CAUSAL, 64>(a, stream);
-  else
+  if (a.D == 128)
     launch_pl_d<T, QK_INT8, CAUSAL, 128>(a, stream);
+  else if (a.kconst && consts_from_lds(a.B * a.H * ((a.N + BM - 1) / BM), CAUSAL, false))
+    launch_pl_d<T, QK_INT8, CAUSAL, 64, false, true>(a, stream);
+  else
+    launch_pl_d<T, QK_INT8, CAUSAL, 64>(a, stream);
 }
 
 template <typename T, bool QK_INT8>
 static void launch_split_t(const AttnArgs& a, hipStream_t stream) {
-  launch_pl_d<T, QK_INT8, false, 64, true>(a, stream);
+  if (consts_from_lds(a.B * a.H * ((a.N + 63) / 64), false, true))
+    launch_pl_d<T, QK_INT8, false, 64, true, true>(a, stream);
+  else
+    launch_pl_d<T, QK_INT8, false, 64, true>(a, stream);
 }
 
 hipError_t launch_attn_fwd_split(const AttnArgs& a, hipStream_t stream) {

@@ -1,12 +1,13 @@
 """Query and output tiles at their edges, and causal grids in every order branch, through every
-main-loop kernel (GPU).
+main-loop kernel; the two forms of the head_dim 64 per-key constants (GPU).
 
 A wave quantizes 32 query rows together (16 or 8 lanes to a row, 4 or 8 rows to a load) and writes
 its output tile in whole row pieces, through LDS; a causal grid starts its tiles longest first, per
 XCD where the planes share out over the 8 XCDs, else over all planes. Row counts around 32 and the
 query tiles, row strides that are no multiple of a row, rows with one large value in any column,
-zero rows; planes below, at and beyond a multiple of 8, with one to many tiles per compute unit.
-Bars: the emulation's; kernels 1-3 bit for bit.
+zero rows; planes below, at and beyond a multiple of 8, with one to many tiles per compute unit. A head_dim 64 launch takes its
+per-key constants from LDS once it has more than 1 (key split), 2 or 3 (causal) blocks for each of
+256 compute units. Bars: the emulation's; kernels 1-3 bit for bit.
 """
 import oracle
 import pytest
@@ -70,3 +71,22 @@ def test_causal_orders_same_bits(B, H, N, D):
     assert torch.isfinite(outs[1]).all()
     for kern, o in outs.items():
         assert torch.equal(o, outs[1]), kern
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("H,N,causal,kern", [
+    (256, 128, False, 3), (257, 128, False, 3), (512, 1, False, 3), (513, 129, False, 3),
+    (171, 300, False, 3), (768, 100, True, 3), (769, 77, True, 3), (257, 321, True, 3),
+    (64, 256, False, 4), (65, 256, False, 4), (257, 33, False, 4), (43, 400, False, 4)])
+def test_d64_constants_same_bits_in_small_and_large_grids(H, N, causal, kern, dtype):
+    # each plane's result is the one it has in a grid of 20 planes, on either side of the line
+    print("case", H, N, causal, kern, dtype, flush=True)
+    q, k, v = (t.cuda() for t in make_qkv(1, H, N, seed=H + N, dtype=dtype, d=64,
+                                          k_offset_std=2.0, v_offset_std=1.0))
+    kw = dict(is_causal=causal, kernel=kern, smooth_v=True, return_lse=True)
+    o, lse = _forward(q, k, v, **kw)
+    assert torch.isfinite(o).all()
+    for h in (0, H - 20):
+        ps = slice(h, h + 20)
+        op, lp = _forward(q[:, ps].contiguous(), k[:, ps].contiguous(), v[:, ps].contiguous(), **kw)
+        assert torch.equal(op, o[:, ps]) and torch.equal(lp, lse[:, ps])
