@@ -8,7 +8,7 @@
 // before, the last plane's longest tiles began when the others had nearly ended.
 // Measured (main loop, us, before / after; fp16, head_dim 128 unless said): 32 heads of 3001 rows
 // 88.1 / 67, 32 of 2048 62.9 / 44.7, 24 of 4096 154.5 / 90, 48 of 1024 35.7 / 26.5, 48 of 8771
-// 718 / 700, head_dim 64, 32 of 4096 165.6 / 89. Calls of few rounds gain most, long ones little
+// 718 / 700, head_dim 64, 32 of 4096 165.6 / 85. Calls of few rounds gain most, long ones little
 // (48 of 16384 2146 / 2127).
 #pragma once
 
