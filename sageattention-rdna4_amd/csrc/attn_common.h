@@ -61,7 +61,7 @@ constexpr int Q_SCRATCH = 32 * 64;
 //   amax = max(max_d |q|, 1e-12); qinv = RN(127/amax) (or 448); q8 = clamp(rne(RN(q*qinv)))
 //   (fp8: e4m3(clamp(RN(q*qinv), +-448))); sq = RN(amax/127) (or 448); c_q = RN(RN(sm*log2e)*sq).
 // The rows are loaded as they lie in memory, D/8 lanes of 16 bytes to a row (4 or 8 whole rows per
-// load), and a row's lanes share the work of its scale (row_max). The bytes reach the MFMA operand
+// load), and a row's lanes share the work of its scale (row_absmax). The bytes reach the MFMA operand
 // layout (lane (q, h): row q, `qf`'s columns) through `scratch`, Q_SCRATCH bytes of LDS of the
 // wave's own, 64 columns at a time. What this replaces, each lane loading its own row and
 // quantizing it alone, touched 64 cache lines per load and took a wave 3.2k cycles of VALU issue:
@@ -85,12 +85,9 @@ __device__ __forceinline__ void quant_q_tile(const T* __restrict__ q, int q0, in
 #pragma unroll
   for (int i = 0; i < NR; ++i)
     w[i] = (row0 + i < N) ? *(const u32x4*)(p + i * q_sr) : (u32x4){0u, 0u, 0u, 0u};
-  float f[NR][8], m[NR];
+  float f[NR][8];
 #pragma unroll
-  for (int i = 0; i < NR; ++i) {
-    unpack8<T>(w[i], f[i]);
-    m[i] = absmax8(f[i]);
-  }
+  for (int i = 0; i < NR; ++i) unpack8<T>(w[i], f[i]);
   if (mu) {
     float v[8], sel = 0.0f;
     const f32x4 m0 = *(const f32x4*)(mu + 8 * cg), m1 = *(const f32x4*)(mu + 8 * cg + 4);
@@ -110,12 +107,7 @@ __device__ __forceinline__ void quant_q_tile(const T* __restrict__ q, int q0, in
     }
     *qmu = __shfl(sel, own, 64);
   }
-  float amax;
-  if constexpr (CG == 16)
-    amax = row_max<16>(m, cg);
-  else
-    amax = row_max(m, cg);
-  amax = fmaxf(amax, SCALE_FLOOR);
+  const float amax = fmaxf(row_absmax<CG>(f, cg), SCALE_FLOOR);
   const float top = QK_INT8 ? I8_MAX : P_SCALE;
   const float qinv = __fdiv_rn(top, amax);
   sq = __shfl(__fdiv_rn(amax, top), own, 64);

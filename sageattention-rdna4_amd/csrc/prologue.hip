@@ -21,7 +21,7 @@
 // Thread layout of both passes: 256 threads = CG = D/8 column groups (cg, 8 columns = one 16-byte
 // load) x RG = 256/CG row groups (rg). In a step of STEP = 8*RG rows a thread holds 8 consecutive
 // rows of 8 columns, so it has 8 consecutive tokens of a column (one 8-byte word of the transposed
-// V tile) and 8 rows whose scales the CG lanes that share them work out together (row_max).
+// V tile) and 8 rows whose scales the CG lanes that share them work out together (row_absmax).
 //
 // What bounds the passes: HBM bandwidth, if enough bytes are in flight and the arithmetic stays
 // out of the way. On gfx950 a wave64 add, multiply, fma, AND or move takes about 2.3 cycles of its
@@ -283,10 +283,7 @@ __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(STATS_BLOCKS
       // the rows' maxima; lane l of the row group gets row l & 7's, and that row's scale
       // sv = max(RN(vmax / 448), 1e-12) and reciprocal: the row's quotients RN(v / sv) come from
       // one correctly rounded reciprocal (div_by: bit-identical to a division per element)
-      float m[8];
-#pragma unroll
-      for (int i = 0; i < 8; ++i) m[i] = absmax8(f[i]);
-      const float vmax = row_max<CG>(m, cg);
+      const float vmax = row_absmax<CG>(f, cg);
       const float sv = fmaxf(div_by(vmax, P_SCALE, RCP_P_SCALE), SCALE_FLOOR);
       const float rsv = __fdiv_rn(1.0f, sv);
       {
@@ -433,11 +430,8 @@ __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(QUANT_BLOCKS
     for (int i = 0; i < 8; ++i)
 #pragma unroll
       for (int e = 0; e < 8; ++e) f[i][e] -= mu[e];
-    float mx[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) mx[i] = absmax8(f[i]);
     // row cg & 7's scale sk = max(RN(kmax / 127 or 448), 1e-12) and reciprocal
-    const float kmax = row_max<CG>(mx, cg);
+    const float kmax = row_absmax<CG>(f, cg);
     const float sk = fmaxf(KINT8 ? div_by(kmax, I8_MAX, RCP_I8_MAX)
                                  : div_by(kmax, P_SCALE, RCP_P_SCALE), SCALE_FLOOR);
     const float rsk = __fdiv_rn(1.0f, sk);

@@ -112,15 +112,26 @@ __device__ __forceinline__ float maxg(float x) {
   return x;
 }
 
-// max(m, |a|, |b|) as one v_max3_f32 (a plain fmaxf of inputs the compiler cannot prove quiet
-// costs a canonicalizing max per input). NaN inputs are ignored, as by fmaxf.
-__device__ __forceinline__ float max3abs(float m, float a, float b) {
+// max(m, |a|, |b|) in one instruction (a plain fmaxf of inputs the compiler cannot prove quiet costs
+// a canonicalizing max per input), NaN if one of them is a NaN. v_max3_f32 would ignore a quiet
+// NaN, as fmaxf does, but returns a NaN for a signalling one and with the next pair loses what came
+// before it; bf16 rows are widened by a shift, which leaves a signalling NaN as it is.
+__device__ __forceinline__ float maximum3abs(float m, float a, float b) {
   float r;
-  asm("v_max3_f32 %0, %1, |%2|, |%3|" : "=v"(r) : "v"(m), "v"(a), "v"(b));
+  asm("v_maximum3_f32 %0, %1, |%2|, |%3|" : "=v"(r) : "v"(m), "v"(a), "v"(b));
   return r;
 }
 __device__ __forceinline__ float absmax8(const float* f) {
-  return max3abs(max3abs(max3abs(max3abs(0.0f, f[0], f[1]), f[2], f[3]), f[4], f[5]), f[6], f[7]);
+  return maximum3abs(
+      maximum3abs(maximum3abs(maximum3abs(0.0f, f[0], f[1]), f[2], f[3]), f[4], f[5]), f[6], f[7]);
+}
+// The same over the values that are no NaN: each is quieted first, and v_max_f32 ignores quiet NaNs.
+__device__ __forceinline__ float absmax8_no_nan(const float* f) {
+  float m = 0.0f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e)
+    asm("v_max_f32 %0, %1, %1\n\tv_max_f32 %0, %2, |%0|" : "=&v"(m) : "v"(f[e]), "v"(m));
+  return m;
 }
 // Non-negative floats order as their bits.
 __device__ __forceinline__ u32 umax(u32 a, u32 b) { return a > b ? a : b; }
@@ -175,6 +186,31 @@ __device__ __forceinline__ float row_max(const float (&m)[4], int lane) {
   u32 o = (u32)__builtin_amdgcn_update_dpp(0, (int)r, 0x104, 0xF, 0x5, false);
   o = (u32)__builtin_amdgcn_update_dpp((int)o, (int)r, 0x114, 0xF, 0xA, false);
   return __uint_as_float(umax(r, o));
+}
+
+// The row absmax of the rows f[0 .. NR-1] (8 columns of each per lane), over the group of CG lanes
+// that share them, NaNs ignored: lane l of the group returns row l % NR's. A NaN in any lane's
+// columns is the largest of the row's bit patterns, so it shows in the result, and a wave that
+// holds one (all its lanes then, the exchange moves data between lanes) works its maxima out again
+// without them.
+template <int CG, int NR>
+__device__ __forceinline__ float row_absmax(const float (&f)[NR][8], int lane) {
+  float m[NR];
+  auto reduce = [&]() {
+    if constexpr (NR == 8)
+      return row_max<CG>(m, lane);
+    else
+      return row_max(m, lane);
+  };
+#pragma unroll
+  for (int i = 0; i < NR; ++i) m[i] = absmax8(f[i]);
+  float r = reduce();
+  if (__builtin_amdgcn_ballot_w64(__float_as_uint(r) > 0x7f800000u) != 0) {
+#pragma unroll
+    for (int i = 0; i < NR; ++i) m[i] = absmax8_no_nan(f[i]);
+    r = reduce();
+  }
+  return r;
 }
 
 // Every lane of a CG-lane group receives lane I (0 .. 7) of its own group.
