@@ -529,6 +529,23 @@ __device__ __forceinline__ void probs_tile(const f32x16 (&x)[2], float w, float 
 // Bytes of LDS a wave needs to write its output tile (store_o_tile): 32 rows x 64 columns of 2 bytes.
 constexpr int O_SCRATCH = 32 * 128;
 
+// T(a * b + c). fp16: rounded once, by v_fma_mixlo_f16, whichever element it is (left to itself the
+// compiler narrows some of the sums from fp32 in pairs, with a second rounding, and which ones
+// depends on the surrounding code; the other half of the word is opaque to it here, so that it
+// cannot pair them). bf16: the fp32 sum narrowed.
+template <typename T>
+__device__ __forceinline__ T fma_narrow(float a, float b, float c) {
+  if constexpr (std::is_same_v<T, f16>) {
+    f16 r = (f16)__builtin_fmaf(a, b, c);
+    asm("" : "+v"(r));
+    return r;
+  } else {
+    float x = __builtin_fmaf(a, b, c);
+    asm("" : "+v"(x));
+    return (T)x;
+  }
+}
+
 // The epilogue: rows q0 .. q0+31 of O = T(acc * inv) (with `vm`, the plane's V mean, T(fma(acc,
 // inv, vm[d]))), inv the lane's own row's factor. The accumulators hold one query per lane, so
 // storing them as they lie writes 16 bytes of each of 32 rows per instruction; they are turned in
@@ -544,15 +561,7 @@ __device__ __forceinline__ void store_o_tile(const f32x16 (&acc)[D / 32], float 
   const int wsw = (l32 >> 1) & 7;
 #pragma unroll
   for (int dd = 0; dd < D / 64; ++dd) {
-    // x is rounded to fp32 before it is narrowed: left to itself the compiler forms some of the
-    // outputs with one rounding (v_fma_mixlo_f16), which ones depending on the surrounding code
-    auto put = [&](int t, int g, float (&x)[4]) {
-      T ov[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        asm("" : "+v"(x[e]));
-        ov[e] = (T)x[e];
-      }
+    auto put = [&](int t, int g, const T (&ov)[4]) {
       u32x2 packed;
       __builtin_memcpy(&packed, ov, 8);
       *(u32x2*)(wr + 16 * ((4 * t + g) ^ wsw)) = packed;
@@ -563,20 +572,25 @@ __device__ __forceinline__ void store_o_tile(const f32x16 (&acc)[D / 32], float 
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
           const f32x4 m = *(const f32x4*)(vm + 64 * dd + 32 * t + 8 * g + 4 * hh);
-          float x[4];
+          T ov[4];
 #pragma unroll
-          for (int e = 0; e < 4; ++e) x[e] = __builtin_fmaf(acc[2 * dd + t][4 * g + e], inv, m[e]);
-          put(t, g, x);
+          for (int e = 0; e < 4; ++e)
+            ov[e] = fma_narrow<T>(acc[2 * dd + t][4 * g + e], inv, m[e]);
+          put(t, g, ov);
         }
     } else {
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
-          float x[4];
+          T ov[4];
 #pragma unroll
-          for (int e = 0; e < 4; ++e) x[e] = acc[2 * dd + t][4 * g + e] * inv;
-          put(t, g, x);
+          for (int e = 0; e < 4; ++e) {
+            float x = acc[2 * dd + t][4 * g + e] * inv;
+            asm("" : "+v"(x));   // the product rounded to fp32, then narrowed, in every kernel
+            ov[e] = (T)x;
+          }
+          put(t, g, ov);
         }
     }
     asm volatile("" ::: "memory");   // the wave's own LDS writes, then its reads, in order
