@@ -117,10 +117,12 @@ __device__ __forceinline__ void unpack_rows(const u32x4 (&w)[8], float (&f)[8][8
   for (int i = 0; i < 8; ++i) unpack8<T>(w[i], f[i]);
 }
 
-// Two tokens' e4m3 bytes of one column into the low (HI = 0) or high half of a word.
+// Two tokens' e4m3 bytes of one column into the low (HI = 0) or high half of a word. The low half
+// is written first: the word has no value before it, and the convert keeps the high half of an
+// operand that the next one overwrites, so a's own bits do (as in fp8x4).
 template <bool HI>
 __device__ __forceinline__ void fp8_pair(u32& w, float a, float b) {
-  w = (u32)__builtin_amdgcn_cvt_pk_fp8_f32(a, b, (int)w, HI);
+  w = (u32)__builtin_amdgcn_cvt_pk_fp8_f32(a, b, HI ? (int)w : __float_as_int(a), HI);
 }
 
 // Sum over c of part[c * D] (c = first, first + step, ...), eight loads in flight at a time.

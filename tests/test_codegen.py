@@ -21,13 +21,13 @@ sys.path.insert(0, PKG)
 
 
 @functools.lru_cache(maxsize=None)
-def _assembly(source):
+def _assembly(source, extra=()):
     import build_lib
     if not os.path.exists(build_lib.HIPCC):
         pytest.skip("hipcc not available")
     flags = [f for f in build_lib.COMMON_FLAGS if f not in ("-fPIC",)]
     flags += build_lib.FILE_FLAGS.get(os.path.basename(source), [])
-    res = subprocess.run([build_lib.HIPCC] + flags + ["--cuda-device-only", "-S", "-o", "-", source],
+    res = subprocess.run([build_lib.HIPCC] + flags + ["--cuda-device-only", "-S", *extra, "-o", "-", source],
                          capture_output=True, text=True)
     assert res.returncode == 0, res.stderr[-2000:]
     return res.stdout
@@ -342,6 +342,44 @@ def test_resource_parser_sees_a_spill():
     meta = ("  - .agpr_count:     0\n    .name:           _Zk\n    .private_segment_fixed_size: 12\n"
             "    .vgpr_count:     168\n    .vgpr_spill_count: 3\n.end_amdgpu_metadata\n")
     assert _kernel_resources(meta) == [("_Zk", 168, 3, 12)]
+
+
+# ---------------------------------------------------------------------------------------------
+# Undefined operands. v_cvt_pk_fp8_f32 writes half a word and keeps the other half of an operand;
+# that operand has to have a value (in the compiler's terms: neither undef nor poison, nor a phi
+# that is one of them on the way into a loop), or the whole result is undefined.
+# ---------------------------------------------------------------------------------------------
+_NO_VALUE = re.compile(r"\b(undef|poison)\b")
+
+
+def undefined_converts(ir):
+    bad = []
+    for fn in re.findall(r"^define .*?^}", ir, re.M | re.S):
+        defs = dict(re.findall(r"^\s*(%[\w.]+) = (.*)$", fn, re.M))
+        for old in re.findall(r"cvt\.pk\.fp8\.f32\([^,]+, [^,]+, i32 (?:noundef )?(\S+), i1", fn):
+            value = defs.get(old, old)
+            if old == value or value.startswith("phi"):
+                if _NO_VALUE.search(value):
+                    bad.append((fn.split("(")[0].split("@")[-1], old, value))
+    return bad
+
+
+def test_undefined_convert_detector():
+    ok = ("define void @k(float %a) {\n  %w = tail call i32 @llvm.amdgcn.cvt.pk.fp8.f32(float %a, "
+          "float %a, i32 0, i1 false)\n}\n")
+    assert undefined_converts(ok) == []
+    assert len(undefined_converts(ok.replace("i32 0", "i32 undef"))) == 1
+    phi = ok.replace("  %w", "  %p = phi i32 [ poison, %e ], [ %w, %l ]\n  %w")
+    assert len(undefined_converts(phi.replace("i32 0", "i32 %p"))) == 1
+
+
+@pytest.mark.parametrize("source", ["prologue.hip", "attn_fwd.hip", "attn_fwd_pp.hip",
+                                    "attn_fwd_pl.hip"])
+def test_fp8_converts_keep_defined_halves(source):
+    ir = _assembly(os.path.join(PKG, "csrc", source), ("-emit-llvm",))
+    assert "cvt.pk.fp8.f32" in ir
+    bad = undefined_converts(ir)
+    assert not bad, bad[:4]
 
 
 # ---------------------------------------------------------------------------------------------
