@@ -382,6 +382,16 @@ def test_fp8_converts_keep_defined_halves(source):
     assert not bad, bad[:4]
 
 
+@pytest.mark.parametrize("source", ["prologue.hip", "attn_fwd.hip", "attn_fwd_pp.hip",
+                                    "attn_fwd_pl.hip"])
+def test_no_flat_accesses(source):
+    # every pointer is to global memory; a flat access also counts as an LDS one, so that every wait
+    # for LDS, for a scalar load or at a barrier would wait for it
+    asm = _assembly(os.path.join(PKG, "csrc", source))
+    assert "global_load" in asm
+    assert re.findall(r"^\s*flat_\w+", asm, re.M) == []
+
+
 # ---------------------------------------------------------------------------------------------
 # Barrier liveness. A workgroup whose waves execute different numbers of `s_barrier` hangs the
 # GPU. In the ping-pong kernel each wave computes up to its own causal diagonal (w_end differs by
