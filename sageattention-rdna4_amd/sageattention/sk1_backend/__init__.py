@@ -45,7 +45,8 @@ ENVELOPE = dict(
 )
 
 _LOGGED = set()
-#: device index -> architecture, which a process's device keeps
+#: device index -> architecture, which a process's device keeps (only calls that name a device by
+#: its index: what "cuda" stands for changes with the current device)
 _ARCHS = {}
 
 
@@ -62,13 +63,16 @@ def device_arch(device=None) -> str:
     (`sageattention/sk1_backend/__init__.py:393-410` of the reference).
     """
     try:
-        index = device.index if isinstance(device, torch.device) else device
-        if index is None:
-            index = torch.cuda.current_device()
-        arch = _ARCHS.get(index)
+        if device is None:
+            device = torch.cuda.current_device()
+        cuda = isinstance(device, torch.device) and device.type == "cuda"
+        index = device.index if cuda else device
+        arch = _ARCHS.get(index) if type(index) is int else None
         if arch is None:
-            name = getattr(torch.cuda.get_device_properties(index), "gcnArchName", "") or ""
-            arch = _ARCHS[index] = name.split(":", 1)[0]
+            name = getattr(torch.cuda.get_device_properties(device), "gcnArchName", "") or ""
+            arch = name.split(":", 1)[0]
+            if arch and type(index) is int:
+                _ARCHS[index] = arch
         return arch
     except Exception:  # noqa: BLE001
         return ""
