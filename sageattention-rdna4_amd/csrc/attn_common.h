@@ -67,7 +67,10 @@ constexpr int Q_SCRATCH = 32 * 64;
 // quantizing it alone, touched 64 cache lines per load and took a wave 3.2k cycles of VALU issue:
 // with one 64-key block per query tile (768 tiles of 128 queries, three per CU) a call took
 // 16.8 us, of which 3.9 us per tile and CU were this and the epilogue.
-// `q`: the plane's row 0. Rows >= N are zero. sq, cq: of the lane's own row q0 + lane % 32.
+// `q`: the plane's row 0. Rows >= N are read as row N-1 (nothing of theirs is written) and every
+// lane's loads are unconditional: between loads under conditions the compiler waits for earlier
+// ones, or for the staging requests ahead of them, a memory latency each time (0.4 of 6.8 us with
+// one key block). sq, cq: of the lane's own row q0 + lane % 32.
 // With `mu` (the plane's smooth_k mean, D fp32), also q . mu of that row in `qmu` (fp32 products
 // and sums, in an order of its own): the row's logsumexp correction for smooth_k.
 template <typename T, bool QK_INT8, int D = HD>
@@ -81,10 +84,12 @@ __device__ __forceinline__ void quant_q_tile(const T* __restrict__ q, int q0, in
   const int own = (l32 / NR) * CG + l32 % NR;   // the lane that works out row l32's scale
   const int row0 = q0 + NR * rg;
   u32x4 w[NR];
-  const T* p = q + (int64_t)row0 * q_sr + 8 * cg;
+  const T* p = q + (int64_t)(row0 < N ? row0 : N - 1) * q_sr + 8 * cg;
 #pragma unroll
-  for (int i = 0; i < NR; ++i)
-    w[i] = (row0 + i < N) ? *(const u32x4*)(p + i * q_sr) : (u32x4){0u, 0u, 0u, 0u};
+  for (int i = 0; i < NR; ++i) {
+    w[i] = *(const u32x4*)p;
+    p += row0 + i + 1 < N ? q_sr : 0;
+  }
   float f[NR][8];
 #pragma unroll
   for (int i = 0; i < NR; ++i) unpack8<T>(w[i], f[i]);

@@ -392,6 +392,26 @@ def test_no_flat_accesses(source):
     assert re.findall(r"^\s*flat_\w+", asm, re.M) == []
 
 
+def q_load_waits(asm):
+    """What stands between the loads of a wave's Q rows (the first 8 vector loads of 16 bytes to
+    registers of a main-loop kernel, 4 at head_dim 64) that a load could wait behind: waits for
+    vector memory and branches."""
+    found = []
+    for name, body in re.findall(r"^(_ZN4sage\w+attn_fwd\w*):(.*?)\.Lfunc_end", asm, re.M | re.S):
+        lines = [l.split(";")[0].strip() for l in body.split("\n")]
+        loads = [i for i, l in enumerate(lines) if re.match(r"global_load_dwordx4 v\[", l)]
+        between = lines[loads[0]:loads[3 if "Li64" in name else 7]]
+        found.append((name, [l for l in between if re.match(r"s_waitcnt.*vmcnt|s_c?branch", l)]))
+    return found
+
+
+@pytest.mark.parametrize("source", ["attn_fwd.hip", "attn_fwd_pp.hip", "attn_fwd_pl.hip"])
+def test_q_rows_are_loaded_together(source):
+    found = q_load_waits(_assembly(os.path.join(PKG, "csrc", source)))
+    assert len(found) >= 6
+    assert [f for f in found if f[1]] == []
+
+
 # ---------------------------------------------------------------------------------------------
 # Barrier liveness. A workgroup whose waves execute different numbers of `s_barrier` hangs the
 # GPU. In the ping-pong kernel each wave computes up to its own causal diagonal (w_end differs by
