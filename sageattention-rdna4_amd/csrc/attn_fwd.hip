@@ -131,6 +131,7 @@ __global__ __launch_bounds__(AT) __attribute__((amdgpu_waves_per_eu(attn_waves(D
                               (u8*)&sB2 + Q_SCRATCH * w, qf, sq, cq,
                               (LSE && KMEAN) ? KMEAN + (int64_t)kvp * D : nullptr, &qmu);
   (void)sq;
+  const float Sb = Sfold[kvp];
   if (LSE && hh == 0) s_qmu[32 * w + l32] = qmu;
 
   f32x16 acc[NDT];
@@ -216,7 +217,6 @@ __global__ __launch_bounds__(AT) __attribute__((amdgpu_waves_per_eu(attn_waves(D
   const int row = q0 + (lane_id() & 31);
   if (LSE && lane_id() < 32 && row < N)
     LSE[(int64_t)bh * N + row] = row_lse(mc, l_i, sm_scale, s_qmu[32 * w + (lane_id() & 31)]);
-  const float Sb = Sfold[kvp];
   const float inv = (l_i > 0.0f) ? __fdiv_rn(Sb, l_i * P_SCALE) : 0.0f;
   store_o_tile<T, D>(acc, inv, VMEAN ? VMEAN + (int64_t)kvp * D : nullptr, O + b * o_sb + hd * o_sh,
                      q0, N, o_sr, (w < 2 ? (u8*)&sB0 : (u8*)&sB1) + O_SCRATCH * (w & 1));

@@ -117,6 +117,7 @@ __global__ __launch_bounds__(PP_T) __attribute__((amdgpu_waves_per_eu(2, 2))) vo
                            (u8*)&sB[2] + Q_SCRATCH * w, qf, sq, cq,
                            (LSE && KMEAN) ? KMEAN + (int64_t)kvp * HD : nullptr, &qmu);
   (void)sq;
+  const float Sb = Sfold[kvp];
 
   f32x16 acc[4];
 #pragma unroll
@@ -317,7 +318,6 @@ __global__ __launch_bounds__(PP_T) __attribute__((amdgpu_waves_per_eu(2, 2))) vo
   const int row = q0 + (lane_id() & 31);
   if (LSE && lane_id() < 32 && row < N)
     LSE[(int64_t)bh * N + row] = row_lse(mc, l_i, sm_scale, qmu);
-  const float Sb = Sfold[kvp];
   const float inv = (l_i > 0.0f) ? __fdiv_rn(Sb, l_i * P_SCALE) : 0.0f;
   store_o_tile<T>(acc, inv, VMEAN ? VMEAN + (int64_t)kvp * HD : nullptr, O + b * o_sb + hd * o_sh,
                   q0, N, o_sr, (u8*)&sB[0] + O_SCRATCH * w);
