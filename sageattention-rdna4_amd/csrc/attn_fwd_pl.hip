@@ -38,6 +38,7 @@
 // The SPLIT form (non-causal head_dim 64, for grids that leave compute units idle) is described
 // at the kernel: 64 queries per block, the key blocks shared out between two wave pairs.
 #include "attn_common.h"
+#include "consts_rule.h"
 #include "sage_launch.h"
 #include "tile_order.h"
 
@@ -414,25 +415,11 @@ static void launch_pl_d(const AttnArgs& a, hipStream_t stream) {
                      a.vmean);
 }
 
-// Where a head_dim 64 softmax takes its per-key constants from (CLDS; same values, same bits). As
-// DPP broadcasts they cost a 4-cycle multiply per score instead of a 2-cycle one; as 16-byte LDS
-// reads that a half-wave shares they cost the read's latency, which only other waves of the SIMD
-// hide. So LDS once a launch keeps several blocks on every CU: main loop, DPP -> LDS, at 1 block
-// per CU 62.7 -> 69.3 us, at 2 92.4 -> 93.1, at 2.5 128.0 -> 123.8, at 4 155.7 -> 153.0
-// (N = 4096), 30 planes of 17550 2591 -> 2514; on a card that throttled under its power cap 6 planes
-// of 32768 went 1809 -> 1836 (1765 -> 1738 on one that did not). A causal launch of fewer than ~3 ends in its longest tiles, each alone on its SIMDs:
-// at 3 63.8 -> 71.3, at 3.5 89.7 -> 84.4, at 4 89.0 -> 85.1. The key split's blocks: at 1
-// 39.3 -> 42.1, at 1.25 18.0 -> 17.8, at 2.5 72.7 -> 69.6. head_dim 128 (three blocks per CU,
-// twice the matrix work a score) gained nothing.
-static bool consts_from_lds(int64_t blocks, bool causal, bool split) {
-  return blocks > 8 * XCD_CUS * (split ? 1 : causal ? 3 : 2);
-}
-
 template <typename T, bool QK_INT8, bool CAUSAL>
 static void launch_pl_t(const AttnArgs& a, hipStream_t stream) {
   if (a.D == 128)
     launch_pl_d<T, QK_INT8, CAUSAL, 128>(a, stream);
-  else if (a.kconst && consts_from_lds(a.B * a.H * ((a.N + BM - 1) / BM), CAUSAL, false))
+  else if (a.kconst && consts_from_lds(a.B * a.H * ((a.N + BM - 1) / BM), a.cus, CAUSAL, false))
     launch_pl_d<T, QK_INT8, CAUSAL, 64, false, true>(a, stream);
   else
     launch_pl_d<T, QK_INT8, CAUSAL, 64>(a, stream);
@@ -440,7 +427,7 @@ static void launch_pl_t(const AttnArgs& a, hipStream_t stream) {
 
 template <typename T, bool QK_INT8>
 static void launch_split_t(const AttnArgs& a, hipStream_t stream) {
-  if (consts_from_lds(a.B * a.H * ((a.N + 63) / 64), false, true))
+  if (consts_from_lds(a.B * a.H * ((a.N + 63) / 64), a.cus, false, true))
     launch_pl_d<T, QK_INT8, false, 64, true, true>(a, stream);
   else
     launch_pl_d<T, QK_INT8, false, 64, true>(a, stream);

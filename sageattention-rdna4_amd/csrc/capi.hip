@@ -384,11 +384,12 @@ int sage_attn_fwd_ex(int dtype, int qk_int8, int causal, const void* q, int64_t 
   a.lse = lse;
   a.kmean = lse ? kmean : nullptr;
   a.vmean = vmean;
-  // SAGE_KERNEL_AUTO: the kernel the grid-fill rule picks for this device (kernel_for)
+  // SAGE_KERNEL_AUTO: the kernel the grid-fill rule picks for this device (kernel_for). A named
+  // kernel needs no CU count: without one its launch assumes 256.
+  rc = cus_of_current_device(&a.cus);
   if (kernel == SAGE_KERNEL_AUTO) {
-    int64_t cus = 0;
-    if ((rc = cus_of_current_device(&cus))) return rc;
-    kernel = kernel_for(B, H, N, D, causal, cus);
+    if (rc) return rc;
+    kernel = kernel_for(B, H, N, D, causal, a.cus);
   }
   if (kernel == SAGE_KERNEL_SPLIT &&
       (rc = check_grid("the key-split main loop", B * H * ((N + 63) / 64), 256)))

@@ -67,6 +67,7 @@ struct AttnArgs {
   float* lse;              // optional (B*H, N) fp32 row logsumexp
   const float* kmean;      // optional (B*H_kv, 128) fp32 smooth_k mean, for the logsumexp correction
   const float* vmean;      // optional (B*H_kv, 128) fp32 smooth_v mean, added to the output
+  int64_t cus = 0;         // compute units of the launch device (<= 0: 256)
 };
 hipError_t launch_attn_fwd(const AttnArgs& a, hipStream_t stream);
 // the two-group ping-pong form of the same main loop (256 queries per block of 8 waves)
