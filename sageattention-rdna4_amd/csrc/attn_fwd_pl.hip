@@ -344,8 +344,9 @@ __global__ __launch_bounds__(AT) __attribute__((amdgpu_waves_per_eu(pl_waves(D, 
     }
     pc = pn;
   }
-  // acc is read below only inside the divergent `qrow < N` branch; keep the loop's MFMAs out
-  // of it (an MFMA under a partial EXEC mask loses the inactive lanes' operand rows).
+  // acc is read from here on: the loop's MFMAs stay ahead of the fence that waits for their results
+  // (and out of the epilogue's branches: an MFMA under a partial EXEC mask loses the inactive lanes'
+  // operand rows).
 #pragma unroll
   for (int dt = 0; dt < NDT; ++dt) keep_live(acc[dt]);
   mfma_result_fence();

@@ -305,8 +305,9 @@ __global__ __launch_bounds__(PP_T) __attribute__((amdgpu_waves_per_eu(2, 2))) vo
     end_phase2();
   }
   if (g == 1 && w_end == j_end) pv_rt(j_end - 1);
-  // acc is read below only inside the divergent `qrow < N` branch; keep every MFMA out of it
-  // (an MFMA under a partial EXEC mask loses the inactive lanes' operand rows).
+  // acc is read from here on: the loop's MFMAs stay ahead of the fence that waits for their results
+  // (and out of the epilogue's branches: an MFMA under a partial EXEC mask loses the inactive lanes'
+  // operand rows).
 #pragma unroll
   for (int dt = 0; dt < 4; ++dt) asm volatile("" ::"v"(acc[dt]));
   mfma_result_fence();

@@ -349,7 +349,7 @@ __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(STATS_BLOCKS
       __syncthreads();
     }
     // block max of sv over live rows
-    float mx = maxg<16>(sv_max);
+    float mx = max_row16(sv_max);
 #pragma unroll
     for (int o = 16; o < 64; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
     if ((tid & 63) == 0) wmax[tid >> 6] = mx;
@@ -401,7 +401,7 @@ __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(QUANT_BLOCKS
   // S = max(1, max sv) and the mean
   float m = 1.0f;
   for (int i = tid; i < (int)C1; i += PT) m = fmaxf(m, smax[bh * C1 + i]);
-  m = maxg<16>(m);
+  m = max_row16(m);
 #pragma unroll
   for (int o = 16; o < 64; o <<= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
   if ((tid & 63) == 0) wmax[tid >> 6] = m;

@@ -3,7 +3,7 @@
 // Numerics rules that every quantizer in this library follows, because the quantized tensors must
 // be bit-exact with the reference scheme:
 //   * fp32 division is correctly rounded (`__fdiv_rn`); the library is never built with fast-math;
-//   * rounding to an integer is round-half-to-even (`rintf` -> v_rndne_f32), then clamped;
+//   * rounding to an integer is round-half-to-even, of values clamped to its range (i8x4);
 //   * fp32 -> e4m3 goes through v_cvt_pk_fp8_f32 (OCP e4m3fn, round-to-nearest-even on gfx950);
 //   * no fused multiply-add is formed where the scheme has two roundings: every such expression has
 //     no addition (a*b*c), so contraction cannot apply.
@@ -55,10 +55,6 @@ __device__ __forceinline__ void unpack8(const u32x4 w, float* out) {
   }
 }
 
-// Two fp32 -> two e4m3 bytes in the low 16 bits (byte 0 = a).
-__device__ __forceinline__ uint32_t fp8x2(float a, float b) {
-  return ((uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(a, b, 0, false)) & 0xffffu;
-}
 // Four fp32 -> four e4m3 bytes, memory order a, b, c, d.
 __device__ __forceinline__ uint32_t fp8x4(float a, float b, float c, float d) {
   // The first convert writes the low half-word and keeps the high half of its "old" operand,
@@ -100,15 +96,14 @@ template <int CTRL>
 __device__ __forceinline__ float dpp_mov(float v) {
   return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, false));
 }
-// Max over the G lanes of an aligned G-lane group (G = 8 or 16: lanes Gg .. Gg+G-1), as DPP
-// moves folded into v_max_f32: xor 1 and xor 2 (quad_perm), then the mirrored lane of the
-// 8-lane half-row (the other quad) and of the 16-lane row (the other half).
-template <int G = 16>
-__device__ __forceinline__ float maxg(float x) {
+// Max over the lanes of each 16-lane row, as DPP moves folded into v_max_f32: xor 1 and xor 2
+// (quad_perm), then the mirrored lane of the 8-lane half-row (the other quad) and of the 16-lane
+// row (the other half).
+__device__ __forceinline__ float max_row16(float x) {
   x = fmaxf(x, dpp_mov<0xB1>(x));    // quad_perm [1,0,3,2]
   x = fmaxf(x, dpp_mov<0x4E>(x));    // quad_perm [2,3,0,1]
   x = fmaxf(x, dpp_mov<0x141>(x));   // row_half_mirror
-  if (G == 16) x = fmaxf(x, dpp_mov<0x140>(x));   // row_mirror
+  x = fmaxf(x, dpp_mov<0x140>(x));   // row_mirror
   return x;
 }
 

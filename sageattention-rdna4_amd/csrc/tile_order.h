@@ -24,7 +24,8 @@
 
 namespace sage {
 
-constexpr int XCDS = 8, XCD_CUS = 32;   // MI355X: 256 CUs in 8 XCDs
+constexpr int XCDS = 8, XCD_CUS = 32;   // MI355X: 256 CUs in 8 XCDs (a partition has fewer XCDs: the
+                                        // eight shares then mix on them, each longest first)
 
 struct CausalTile {
   int bh;     // plane
