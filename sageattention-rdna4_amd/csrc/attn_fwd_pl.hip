@@ -78,7 +78,7 @@ __global__ __launch_bounds__(AT) __attribute__((amdgpu_waves_per_eu(pl_waves(D, 
     int64_t sk_plane, int64_t sk_block, const float* __restrict__ Wr, int64_t w_plane,
     int64_t w_block, float w_mul, const u8* __restrict__ V8T, const float* __restrict__ Sfold,
     T* __restrict__ O, int64_t q_sb, int64_t q_sh, int64_t q_sr, int64_t o_sb, int64_t o_sh,
-    int64_t o_sr, int H, int H_kv, int G, int N, int Nk, int Nk_pad, int num_qt, int blocks,
+    int64_t o_sr, int H, int H_kv, int G, int N, int Nk, int Nk_pad, int num_qt, int xcd_span,
     float sm_scale, float* __restrict__ LSE, const float* __restrict__ KMEAN,
     const float* __restrict__ VMEAN) {
   static_assert(!(SPLIT && (CAUSAL || D != 64)), "the key split serves non-causal head_dim 64");
@@ -100,12 +100,12 @@ __global__ __launch_bounds__(AT) __attribute__((amdgpu_waves_per_eu(pl_waves(D, 
   // ---- which (plane, q-tile) this block runs: XCD-contiguous planes, longest causal tiles first
   int bh, qt;
   if (CAUSAL) {
-    const CausalTile t = causal_tile(blockIdx.x, blocks, num_qt, pl_waves(D, SPLIT));
+    const CausalTile t = causal_tile(blockIdx.x, xcd_span, num_qt, pl_waves(D, SPLIT));
     bh = t.bh;
     qt = num_qt - 1 - t.rank;
   } else {
     int id = blockIdx.x;
-    if (id < (blocks & ~7)) id = (id & 7) * (blocks >> 3) + (id >> 3);
+    if (id < xcd_span) id = (id & 7) * (xcd_span >> 3) + (id >> 3);
     bh = id / num_qt;
     qt = id - bh * num_qt;
   }
@@ -402,6 +402,7 @@ static void launch_pl_d(const AttnArgs& a, hipStream_t stream) {
   const int BH = (int)(a.B * a.H);
   const int num_qt = (int)((a.N + (SPLIT ? 64 : BM) - 1) / (SPLIT ? 64 : BM));
   const int total = num_qt * BH;
+  const int span = CAUSAL ? total : total / 8 * 8;   // the blocks that the order is over
   // per-key constant rows: the reference's SK / SV' arrays, or the prologue's KCONST layout
   const bool kc = a.kconst != nullptr;
   const float* skr = kc ? a.kconst : a.sk;
@@ -412,7 +413,7 @@ static void launch_pl_d(const AttnArgs& a, hipStream_t stream) {
                      (const T*)a.q, (const u8*)a.k8, skr, plane, blk, wr, plane, blk,
                      kc ? 1.0f : P_SCALE, (const u8*)a.v8t, a.s, (T*)a.o, a.q_sb, a.q_sh, a.q_sr,
                      a.o_sb, a.o_sh, a.o_sr, (int)a.H, (int)a.H_kv, (int)(a.H / a.H_kv), (int)a.N,
-                     (int)a.N_kv, (int)a.N_kv_pad, num_qt, total, a.sm_scale, a.lse, a.kmean,
+                     (int)a.N_kv, (int)a.N_kv_pad, num_qt, span, a.sm_scale, a.lse, a.kmean,
                      a.vmean);
 }
 

@@ -43,7 +43,7 @@ __global__ __launch_bounds__(PP_T) __attribute__((amdgpu_waves_per_eu(2, 2))) vo
     const T* __restrict__ Q, const u8* __restrict__ K8, const float* __restrict__ KC,
     const u8* __restrict__ V8T, const float* __restrict__ Sfold, T* __restrict__ O, int64_t q_sb,
     int64_t q_sh, int64_t q_sr, int64_t o_sb, int64_t o_sh, int64_t o_sr, int H, int H_kv, int G,
-    int N, int Nk, int Nk_pad, int num_qt, int blocks, float sm_scale,
+    int N, int Nk, int Nk_pad, int num_qt, int xcd_span, float sm_scale,
     float* __restrict__ LSE, const float* __restrict__ KMEAN,
     const float* __restrict__ VMEAN) {
   __shared__ StageBuf<HD> sB[3];
@@ -54,12 +54,12 @@ __global__ __launch_bounds__(PP_T) __attribute__((amdgpu_waves_per_eu(2, 2))) vo
   // ---- which (plane, q-tile) this block runs: XCD-contiguous planes, longest causal tiles first
   int bh, qt;
   if (CAUSAL) {
-    const CausalTile t = causal_tile(blockIdx.x, blocks, num_qt, 1);
+    const CausalTile t = causal_tile(blockIdx.x, xcd_span, num_qt, 1);
     bh = t.bh;
     qt = num_qt - 1 - t.rank;
   } else {
     int id = blockIdx.x;
-    if (id < (blocks & ~7)) id = (id & 7) * (blocks >> 3) + (id >> 3);
+    if (id < xcd_span) id = (id & 7) * (xcd_span >> 3) + (id >> 3);
     bh = id / num_qt;
     qt = id - bh * num_qt;
   }
@@ -329,10 +329,11 @@ static void launch_pp_t(const AttnArgs& a, hipStream_t stream) {
   const int BH = (int)(a.B * a.H);
   const int num_qt = (int)((a.N + PP_BM - 1) / PP_BM);
   const int total = num_qt * BH;
+  const int span = CAUSAL ? total : total / 8 * 8;   // the blocks that the order is over
   hipLaunchKernelGGL((attn_fwd_pp_kernel<T, QK_INT8, CAUSAL>), dim3(total), dim3(PP_T), 0, stream,
                      (const T*)a.q, (const u8*)a.k8, a.kconst, (const u8*)a.v8t, a.s, (T*)a.o,
                      a.q_sb, a.q_sh, a.q_sr, a.o_sb, a.o_sh, a.o_sr, (int)a.H, (int)a.H_kv,
-                     (int)(a.H / a.H_kv), (int)a.N, (int)a.N_kv, (int)a.N_kv_pad, num_qt, total,
+                     (int)(a.H / a.H_kv), (int)a.N, (int)a.N_kv, (int)a.N_kv_pad, num_qt, span,
                      a.sm_scale, a.lse, a.kmean, a.vmean);
 }
 
