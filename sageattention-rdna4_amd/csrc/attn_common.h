@@ -180,9 +180,11 @@ __device__ __forceinline__ uint32_t lds_addr(const void* p) {
 // for them (the caller's s_waitcnt does, before the barrier that publishes the data) nor spends
 // per-lane 64-bit adds on the addresses. Any of its own vector-memory waits stay correct: the
 // counter retires in order, so extra operations in flight only make its waits longer.
+// OFF (below 4096) is added to both the global and the LDS address.
+template <int OFF = 0>
 __device__ __forceinline__ void dma16(const void* base, uint32_t voff, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-               :: "v"(voff), "s"(base), "s"(lds) : "memory", "m0");
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 offset:%3"
+               :: "v"(voff), "s"(base), "s"(lds), "n"(OFF) : "memory", "m0");
 }
 __device__ __forceinline__ void dma4(const void* base, uint32_t voff, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1"

@@ -99,7 +99,8 @@ __global__ __launch_bounds__(AT) __attribute__((amdgpu_waves_per_eu(attn_waves(D
   //   KC:  waves 0 and 1 carry floats 64w..64w+63 of the block's 128 (4 B/lane); waves 2 and 3
   //        repeat them into the tile's pad.
   // A wave's second request of a tile lies a whole number of swizzle periods on (8 or 16 rows of K,
-  // 16 of V^T), so it has the first one's per-lane offset from a base of its own.
+  // 16 of V^T), so it has the first one's per-lane offset: K's 1 KB further in memory as in LDS, an
+  // immediate offset, V^T's from a base of its own.
   const int krow = (1024 / D) * NKV * w + lane / (D / 16), kpos = lane % (D / 16);
   const uint32_t k_off = (uint32_t)(krow * D + 16 * (kpos ^ kswz<D>(krow)));
   const int vd = 16 * NKV * w + (lane >> 2), vpos = lane & 3;
@@ -111,8 +112,8 @@ __global__ __launch_bounds__(AT) __attribute__((amdgpu_waves_per_eu(attn_waves(D
     const u8* vblk = Vb + (size_t)BK * (uint32_t)j;
     const u8* cblk = (const u8*)KCb + (size_t)(128 * 4) * (uint32_t)j;
     const uint32_t kl = lds_addr(buf.k) + 1024 * NKV * w, vl = lds_addr(buf.v) + 1024 * NKV * w;
-#pragma unroll
-    for (int i = 0; i < NKV; ++i) dma16(kblk + 1024 * i, k_off, kl + 1024 * i);
+    dma16(kblk, k_off, kl);
+    if constexpr (NKV == 2) dma16<1024>(kblk, k_off, kl);
 #pragma unroll
     for (int i = 0; i < NKV; ++i) dma16(vblk + (size_t)(16 * i) * (uint32_t)Nk_pad, v_off, vl + 1024 * i);
     dma4(cblk, c_off, lds_addr(&buf.s) + c_dst);

@@ -142,7 +142,8 @@ __global__ __launch_bounds__(AT) __attribute__((amdgpu_waves_per_eu(pl_waves(D, 
   // ---- staging: per block every wave issues NKV KB of K and NKV KB of V^T; waves 0 and 1 also
   // 256 bytes of constants (SK, W). Layouts as in attn_fwd.hip.
   // A wave's second request of a tile lies a whole number of swizzle periods on (8 or 16 rows of K,
-  // 16 of V^T), so it has the first one's per-lane offset from a base of its own.
+  // 16 of V^T), so it has the first one's per-lane offset: K's 1 KB further in memory as in LDS, an
+  // immediate offset, V^T's from a base of its own.
   const int krow = (1024 / D) * NKV * ws + lane / (D / 16), kpos = lane % (D / 16);
   const uint32_t k_off = (uint32_t)(krow * D + 16 * (kpos ^ kswz<D>(krow)));
   const int vd = 16 * NKV * ws + (lane >> 2), vpos = lane & 3;
@@ -152,8 +153,8 @@ __global__ __launch_bounds__(AT) __attribute__((amdgpu_waves_per_eu(pl_waves(D, 
     const u8* kblk = Kb + (size_t)(KS * BK * D) * (uint32_t)j;
     const u8* vblk = Vb + (size_t)(KS * BK) * (uint32_t)j;
     const uint32_t kl = lds_addr(buf.k) + 1024 * NKV * ws, vl = lds_addr(buf.v) + 1024 * NKV * ws;
-#pragma unroll
-    for (int i = 0; i < NKV; ++i) dma16(kblk + 1024 * i, k_off, kl + 1024 * i);
+    dma16(kblk, k_off, kl);
+    if constexpr (NKV == 2) dma16<1024>(kblk, k_off, kl);
 #pragma unroll
     for (int i = 0; i < NKV; ++i) dma16(vblk + (size_t)(16 * i) * (uint32_t)Nk_pad, v_off, vl + 1024 * i);
     if (ws < 2) dma4(Cb, c_off + c_blk * (uint32_t)j, lds_addr(ws == 0 ? buf.c.sk : buf.c.w));
