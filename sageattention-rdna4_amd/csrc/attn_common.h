@@ -112,7 +112,7 @@ __device__ __forceinline__ void quant_q_tile(const T* __restrict__ q, int q0, in
     }
     *qmu = __shfl(sel, own, 64);
   }
-  const float amax = fmaxf(row_absmax<CG>(f, cg), SCALE_FLOOR);
+  const float amax = fmaxf(row_absmax<CG, std::is_same_v<T, f16>>(f, cg), SCALE_FLOOR);
   const float top = QK_INT8 ? I8_MAX : P_SCALE;
   const float qinv = __fdiv_rn(top, amax);
   sq = __shfl(__fdiv_rn(amax, top), own, 64);

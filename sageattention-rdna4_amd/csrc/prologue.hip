@@ -290,7 +290,7 @@ __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(STATS_BLOCKS
       // the rows' maxima; lane l of the row group gets row l & 7's, and that row's scale
       // sv = max(RN(vmax / 448), 1e-12) and reciprocal: the row's quotients RN(v / sv) come from
       // one correctly rounded reciprocal (div_by: bit-identical to a division per element)
-      const float vmax = row_absmax<CG>(f, cg);
+      const float vmax = row_absmax<CG, VMODE == V_CENTERED || std::is_same_v<T, f16>>(f, cg);
       const float sv = fmaxf(div_by(vmax, P_SCALE, RCP_P_SCALE), SCALE_FLOOR);
       const float rsv = __fdiv_rn(1.0f, sv);
       {
@@ -441,7 +441,7 @@ __global__ __launch_bounds__(PT) __attribute__((amdgpu_waves_per_eu(QUANT_BLOCKS
 #pragma unroll
       for (int e = 0; e < 8; ++e) f[i][e] -= mu[e];
     // row cg & 7's scale sk = max(RN(kmax / 127 or 448), 1e-12) and reciprocal
-    const float kmax = row_absmax<CG>(f, cg);
+    const float kmax = row_absmax<CG, true>(f, cg);
     const float sk = fmaxf(KINT8 ? div_by(kmax, I8_MAX, RCP_I8_MAX)
                                  : div_by(kmax, P_SCALE, RCP_P_SCALE), SCALE_FLOOR);
     const float rsk = __fdiv_rn(1.0f, sk);

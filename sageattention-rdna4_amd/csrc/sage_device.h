@@ -108,19 +108,28 @@ __device__ __forceinline__ float max_row16(float x) {
 }
 
 // max(m, |a|, |b|) in one instruction (a plain fmaxf of inputs the compiler cannot prove quiet costs
-// a canonicalizing max per input), NaN if one of them is a NaN. v_max3_f32 would ignore a quiet
-// NaN, as fmaxf does, but returns a NaN for a signalling one and with the next pair loses what came
-// before it; bf16 rows are widened by a shift, which leaves a signalling NaN as it is.
+// a canonicalizing max per input). Quiet NaNs are ignored, as by fmaxf; for a signalling one the
+// result is a NaN, and the maximum before it is lost with the next pair.
+__device__ __forceinline__ float max3abs(float m, float a, float b) {
+  float r;
+  asm("v_max3_f32 %0, %1, |%2|, |%3|" : "=v"(r) : "v"(m), "v"(a), "v"(b));
+  return r;
+}
+// The same, but NaN if one of them is a NaN of either kind.
 __device__ __forceinline__ float maximum3abs(float m, float a, float b) {
   float r;
   asm("v_maximum3_f32 %0, %1, |%2|, |%3|" : "=v"(r) : "v"(m), "v"(a), "v"(b));
   return r;
 }
+template <bool QUIET>
 __device__ __forceinline__ float absmax8(const float* f) {
-  return maximum3abs(
-      maximum3abs(maximum3abs(maximum3abs(0.0f, f[0], f[1]), f[2], f[3]), f[4], f[5]), f[6], f[7]);
+  float m = 0.0f;
+#pragma unroll
+  for (int e = 0; e < 8; e += 2)
+    m = QUIET ? max3abs(m, f[e], f[e + 1]) : maximum3abs(m, f[e], f[e + 1]);
+  return m;
 }
-// The same over the values that are no NaN: each is quieted first, and v_max_f32 ignores quiet NaNs.
+// Over the values that are no NaN: each is quieted first, and v_max_f32 ignores quiet NaNs.
 __device__ __forceinline__ float absmax8_no_nan(const float* f) {
   float m = 0.0f;
 #pragma unroll
@@ -184,11 +193,13 @@ __device__ __forceinline__ float row_max(const float (&m)[4], int lane) {
 }
 
 // The row absmax of the rows f[0 .. NR-1] (8 columns of each per lane), over the group of CG lanes
-// that share them, NaNs ignored: lane l of the group returns row l % NR's. A NaN in any lane's
-// columns is the largest of the row's bit patterns, so it shows in the result, and a wave that
-// holds one (all its lanes then, the exchange moves data between lanes) works its maxima out again
-// without them.
-template <int CG, int NR>
+// that share them, NaNs ignored: lane l of the group returns row l % NR's.
+// QUIET: the values hold no signalling NaN (the result of an operation or of an fp16 -> fp32
+// conversion; a bf16 widened by a shift may be one). Otherwise the maxima keep NaNs: one in any
+// lane's columns is the largest of the row's bit patterns, so it shows in the result, and a wave
+// that holds one (all its lanes then, the exchange moves data between lanes) works its maxima out
+// again without them.
+template <int CG, bool QUIET, int NR>
 __device__ __forceinline__ float row_absmax(const float (&f)[NR][8], int lane) {
   float m[NR];
   auto reduce = [&]() {
@@ -198,9 +209,9 @@ __device__ __forceinline__ float row_absmax(const float (&f)[NR][8], int lane) {
       return row_max(m, lane);
   };
 #pragma unroll
-  for (int i = 0; i < NR; ++i) m[i] = absmax8(f[i]);
+  for (int i = 0; i < NR; ++i) m[i] = absmax8<QUIET>(f[i]);
   float r = reduce();
-  if (__builtin_amdgcn_ballot_w64(__float_as_uint(r) > 0x7f800000u) != 0) {
+  if (!QUIET && __builtin_amdgcn_ballot_w64(__float_as_uint(r) > 0x7f800000u) != 0) {
 #pragma unroll
     for (int i = 0; i < NR; ++i) m[i] = absmax8_no_nan(f[i]);
     r = reduce();
