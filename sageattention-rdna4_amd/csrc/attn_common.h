@@ -90,6 +90,9 @@ __device__ __forceinline__ void quant_q_tile(const T* __restrict__ q, int q0, in
     w[i] = *(const u32x4*)p;
     p += row0 + i + 1 < N ? q_sr : 0;
   }
+  // no row is unpacked before the last one is requested (left to itself the compiler waits for the
+  // first row ahead of the eighth's request in some instances)
+  __builtin_amdgcn_sched_barrier(0);
   float f[NR][8];
 #pragma unroll
   for (int i = 0; i < NR; ++i) unpack8<T>(w[i], f[i]);
