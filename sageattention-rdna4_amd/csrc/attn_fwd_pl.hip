@@ -251,6 +251,14 @@ __global__ __launch_bounds__(AT) __attribute__((amdgpu_waves_per_eu(pl_waves(D, 
     kw1 = buf.c.w[c + 16];
   };
   if constexpr (!CLDS) load_consts(sB[0]);
+  // Where the loop starts within 32 bytes of code decides how its instructions fall into fetches, which
+  // a wave alone on its SIMD feels: the same loop at 0, 8, 16 and 24 bytes past such a boundary takes
+  // 76.0, 76.0, 77.4 and 75.5 us (8 planes of 4096; 32 heads of 1 row on 4096 keys 71.1, 71.1, 71.7
+  // and 70.6; e4m3 scores 71.9, 72.1, 72.8 and 71.0), again the same 32 bytes on. Left to the length
+  // of the code before it, it moves with every change there. head_dim 64 (no padding / 24 bytes): 30
+  // planes of 17550 2524 / 2530, the key split 68.8 / 68.9, causal 63.6 / 62.6 (int8) and 59.3 / 60.0
+  // (e4m3). (Some instances park a register between here and the loop: 8 bytes more.)
+  asm volatile(".p2align 5\n\t.rept %0\n\ts_nop 0\n\t.endr" ::"n"(D == 128 ? 6 : 0));
   for (int j = 0;; ++j) {   // ends at j == j_end, after that iteration's P.V
     const int pm = pc == 0 ? 2 : pc - 1, pn = pc == 2 ? 0 : pc + 1;
     PlBuf<D>& bprev = sB[pm];

@@ -412,6 +412,23 @@ def test_q_rows_are_loaded_together(source):
     assert [f for f in found if f[1]] == []
 
 
+def test_pipelined_loops_start_at_their_place():
+    # the padding that places the loop in its instruction fetches stands right before the loop (at
+    # most a parked register between), once in each kernel
+    asm = _assembly(os.path.join(PKG, "csrc", "attn_fwd_pl.hip"))
+    kernels = re.findall(r"^(_ZN4sage\w+attn_fwd_pl\w*):(.*?)\.Lfunc_end", asm, re.M | re.S)
+    assert len(kernels) >= 12
+    for name, body in kernels:
+        parts = body.split("\t.p2align 5\n")
+        assert len(parts) == 2, name
+        after = [l.split(";")[0].strip() for l in parts[1].split(".endr", 1)[1].split("\n")]
+        after = [l for l in after if l]
+        at = next(i for i, l in enumerate(after) if l.startswith(".LBB"))
+        assert at <= 1, (name, after[:at])
+        label = after[at].rstrip(":")
+        assert any(re.match(r"s_c?branch\w*\s+%s$" % re.escape(label), l) for l in after[at + 1:]), name
+
+
 # ---------------------------------------------------------------------------------------------
 # Barrier liveness. A workgroup whose waves execute different numbers of `s_barrier` hangs the
 # GPU. In the ping-pong kernel each wave computes up to its own causal diagonal (w_end differs by
