@@ -192,6 +192,12 @@ int kernel_for(int64_t B, int64_t H, int64_t N, int64_t D, int causal, int64_t c
     return (!causal && nb64 <= 6 * cus) ? SAGE_KERNEL_SPLIT : SAGE_KERNEL_PIPE;
   }
   const int64_t nb256 = B * H * ((N + 255) / 256);
+  // Causal: the ping-pong from 4 of its blocks per CU on, but for lengths that it pads much more.
+  // Main loop on 256 CUs, ping-pong / pipelined, us: fp16 30 x 8192 (3.75 per CU) 398 / 386, 60 x 4096
+  // (3.75) 223 / 213, 16 x 16384 (4) 785 / 773, 48 x 16384 (12) 2437 / 2397; bf16 30 x 8192 358 / 357,
+  // 16 x 16384 718 / 738, 48 x 8192 (6) 577 / 595, 48 x 16384 2276 / 2227. So the line is right to a
+  // few percent for long planes; with many short ones the pipelined kernel's finer tiles stay ahead
+  // (fp16 250 x 2048 297 / 271, 100 x 4000 400 / 373), which the rule does not know.
   if (causal)
     return (nb256 >= 4 * cus && causal_pad_work(N, 256) - causal_pad_work(N, 128) < 0.02)
                ? SAGE_KERNEL_Q256
