@@ -604,11 +604,19 @@ __device__ __forceinline__ void store_o_tile(const f32x16 (&acc)[D / 32], float 
         }
     }
     asm volatile("" ::: "memory");   // the wave's own LDS writes, then its reads, in order
+    const int r0 = lane >> 3, c = lane & 7;
+    u32x4 x[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      const int r = 8 * k + (lane >> 3), c = lane & 7;
-      const u32x4 x = *(const u32x4*)(scratch + 128 * r + 16 * (c ^ ((r >> 1) & 7)));
-      if (q0 + r < N) *(u32x4*)(o + (int64_t)(q0 + r) * o_sr + 64 * dd + 8 * c) = x;
+      const int r = 8 * k + r0;
+      x[k] = *(const u32x4*)(scratch + 128 * r + 16 * (c ^ ((r >> 1) & 7)));
+    }
+    // all four reads before the first row's condition: behind it each would wait by itself
+    asm volatile("" : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]));
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int r = q0 + 8 * k + r0;
+      if (r < N) *(u32x4*)(o + (int64_t)r * o_sr + 64 * dd + 8 * c) = x[k];
     }
     asm volatile("" ::: "memory");
   }
