@@ -211,7 +211,7 @@ __device__ __forceinline__ float row_absmax(const float (&f)[NR][8], int lane) {
 #pragma unroll
   for (int i = 0; i < NR; ++i) m[i] = absmax8<QUIET>(f[i]);
   float r = reduce();
-  if (!QUIET && __builtin_amdgcn_ballot_w64(__float_as_uint(r) > 0x7f800000u) != 0) {
+  if (!QUIET && __builtin_expect(__builtin_amdgcn_ballot_w64(__float_as_uint(r) > 0x7f800000u) != 0, 0)) {
 #pragma unroll
     for (int i = 0; i < NR; ++i) m[i] = absmax8_no_nan(f[i]);
     r = reduce();

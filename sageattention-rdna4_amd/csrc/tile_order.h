@@ -40,8 +40,9 @@ SAGE_HD CausalTile causal_tile(int block, int blocks, int num_qt, int resident) 
   const unsigned x = u % XCDS;
   unsigned i = u / XCDS;                             // the XCD's i-th block
   const unsigned per = (unsigned)blocks / XCDS;      // blocks of an XCD, or one more
-  if (per <= XCD_CUS) {
-    // A CU for each block: the order does not matter, so planes stay together.
+  if (__builtin_expect(per <= XCD_CUS, 1)) {
+    // A CU for each block: the order does not matter, so planes stay together. (The branch that is
+    // expected, so that these calls run straight on: instructions are fetched anew in a short one.)
     const unsigned id = u < per * XCDS ? x * per + i : u;
     const unsigned bh = id / qt;
     return {(int)bh, (int)(id - bh * qt)};
