@@ -561,7 +561,11 @@ __device__ __forceinline__ T fma_narrow(float a, float b, float c) {
 // storing them as they lie writes 16 bytes of each of 32 rows per instruction; they are turned in
 // `scratch` (O_SCRATCH bytes of LDS of the wave's own) 64 columns at a time and go out as whole
 // 128-byte row pieces, 8 rows per store.
-template <typename T, int D = HD>
+// TOGETHER: the four reads of 64 columns wait together; otherwise each stands behind its row's
+// condition and waits by itself. Pipelined kernel, causal 48 planes of 64 rows 6.77 -> 6.59 us, 24
+// planes of 8771 rows on 512 keys 59.9 -> 59.4; the ping-pong kernel was slower with it (48 planes of
+// 1024 rows 30.1 -> 30.4, 8 of 8192 187.8 -> 188.8: its main loops come out otherwise).
+template <typename T, int D = HD, bool TOGETHER = true>
 __device__ __forceinline__ void store_o_tile(const f32x16 (&acc)[D / 32], float inv,
                                              const float* __restrict__ vm, T* __restrict__ o,
                                              int q0, int N, int64_t o_sr, u8* scratch) {
@@ -605,18 +609,22 @@ __device__ __forceinline__ void store_o_tile(const f32x16 (&acc)[D / 32], float 
     }
     asm volatile("" ::: "memory");   // the wave's own LDS writes, then its reads, in order
     const int r0 = lane >> 3, c = lane & 7;
-    u32x4 x[4];
+    auto read = [&](int r) {
+      return *(const u32x4*)(scratch + 128 * r + 16 * (c ^ ((r >> 1) & 7)));
+    };
+    auto write = [&](int r, u32x4 x) {
+      if (q0 + r < N) *(u32x4*)(o + (int64_t)(q0 + r) * o_sr + 64 * dd + 8 * c) = x;
+    };
+    if constexpr (TOGETHER) {
+      u32x4 x[4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const int r = 8 * k + r0;
-      x[k] = *(const u32x4*)(scratch + 128 * r + 16 * (c ^ ((r >> 1) & 7)));
-    }
-    // all four reads before the first row's condition: behind it each would wait by itself
-    asm volatile("" : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]));
+      for (int k = 0; k < 4; ++k) x[k] = read(8 * k + r0);
+      asm volatile("" ::: "memory");   // the reads are requested ahead of the first row's condition
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const int r = q0 + 8 * k + r0;
-      if (r < N) *(u32x4*)(o + (int64_t)r * o_sr + 64 * dd + 8 * c) = x[k];
+      for (int k = 0; k < 4; ++k) write(8 * k + r0, x[k]);
+    } else {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) write(8 * k + r0, read(8 * k + r0));
     }
     asm volatile("" ::: "memory");
   }

@@ -320,8 +320,8 @@ __global__ __launch_bounds__(PP_T) __attribute__((amdgpu_waves_per_eu(2, 2))) vo
   if (LSE && lane_id() < 32 && row < N)
     LSE[(int64_t)bh * N + row] = row_lse(mc, l_i, sm_scale, qmu);
   const float inv = (l_i > 0.0f) ? __fdiv_rn(Sb, l_i * P_SCALE) : 0.0f;
-  store_o_tile<T>(acc, inv, VMEAN ? VMEAN + (int64_t)kvp * HD : nullptr, O + b * o_sb + hd * o_sh,
-                  q0, N, o_sr, (u8*)&sB[0] + O_SCRATCH * w);
+  store_o_tile<T, HD, false>(acc, inv, VMEAN ? VMEAN + (int64_t)kvp * HD : nullptr,
+                             O + b * o_sb + hd * o_sh, q0, N, o_sr, (u8*)&sB[0] + O_SCRATCH * w);
 }
 
 template <typename T, bool QK_INT8, bool CAUSAL>
